@@ -51,3 +51,21 @@ def test_adapter_term_with_a_factor_off_sixteen_bytes(device, oracle, shift):
     got = Q.QloraLinear(lin, ad).forward(xt).cpu().numpy().astype(np.float64)
     bound = (np.abs(x) @ np.abs(a)) @ np.abs(b) * s
     assert float(np.max(np.abs(got - oracle.lora_ref_f64(x, a, b, s)) / bound)) <= TOL_F32
+
+
+def test_rows_past_one_launch(device):
+    """2^24 + 3 rows through an adapted f32 linear of 4 inputs: a launch of a
+    1024-thread workgroup per four rows would pass 2^32 work items, which wrap."""
+    K, N, r, s, M = 4, 4, 1, 2.0, (1 << 24) + 3
+    g = torch.Generator(device)
+    g.manual_seed(0x95)
+    w, a, b = [torch.randn(*d, generator=g, device=device) for d in ((K, N), (K, r), (r, N))]
+    x = torch.randn(M, K, generator=g, device=device)
+    layer = Q.QLoRALinear(Q.DenseLinear(w), Q.LoraAdapter.from_parts(a, b, s), K * N, False)
+    y = layer.forward(x)
+    # f32 sums of K products and of one more: 1e-5 of the sum of |products|
+    for m in range(0, M, 1 << 22):
+        xm = x[m:m + (1 << 22)].double()
+        ref = xm @ w.double() + (xm @ a.double()) @ b.double() * s
+        bound = xm.abs() @ w.double().abs() + (xm.abs() @ a.double().abs()) @ b.double().abs() * s
+        assert float(((y[m:m + (1 << 22)].double() - ref).abs() / bound).max()) <= TOL_F32, m

@@ -20,6 +20,8 @@
 //     gradients).
 #include "nf4_generic.hpp"
 
+#include <algorithm>
+
 namespace unifur {
 namespace {
 
@@ -106,7 +108,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const void* __restrict__ 
 // workgroups (no scratch, no hand-off, one order of the sum).  A lane owns
 // VEC columns of one k; LPK lanes (a power of two) cover the rank and the
 // wave 64 / LPK consecutive k, so a factor load is one contiguous run per
-// wave; kXaDepth steps of the wave are in flight together.  The k of a wave
+// wave; D steps of the wave are in flight together.  The k of a wave
 // are summed across its lanes, then the 16 waves through LDS.
 // The form before had one thread walk all of K, one dependent load pair at a
 // time: an adapted 4096 -> 4096 linear took 956 us at 1 row and 1002 us at 64
@@ -187,10 +189,20 @@ void launch_xa(const void* x, const float* a, int M, int K, int rank, size_t sk,
   // rows 19.0 us against 24.0 with four rows a workgroup, 64 rows 43 against
   // 48; 4096 -> 4096 at 100 rows 25.7 against 30).  Past that, four rows share
   // each factor load.
-  if (M <= 256)
+  if (M <= 256) {
     lora_xa_kernel<XBF16, VEC, 1><<<M, kXaThreads, 0, stream>>>(x, a, M, K, rank, lpk, sk, sj, xa);
-  else
-    lora_xa_kernel<XBF16, VEC, 4><<<(M + 3) / 4, kXaThreads, 0, stream>>>(x, a, M, K, rank, lpk, sk, sj, xa);
+    return;
+  }
+  // at most kXaRows rows a launch: the work items of one past 2^32 wrap
+  // without an error
+  constexpr int kXaRows = 1 << 23;
+  static_assert((uint64_t)kXaRows / 4 * kXaThreads < 1ull << 32, "work items of a launch");
+  for (int64_t m = 0; m < M; m += kXaRows) {
+    const int rows = (int)std::min<int64_t>(kXaRows, M - m);
+    const void* xm = static_cast<const char*>(x) + (size_t)m * K * (XBF16 ? 2 : 4);
+    lora_xa_kernel<XBF16, VEC, 4><<<(rows + 3) / 4, kXaThreads, 0, stream>>>(xm, a, rows, K, rank, lpk, sk, sj,
+                                                                          xa + (size_t)m * rank);
+  }
 }
 
 __global__ void silu_mul_kernel(const float* __restrict__ g, const float* __restrict__ u, size_t n,
