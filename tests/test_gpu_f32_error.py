@@ -1,0 +1,67 @@
+"""Rounding error of the f32 GEMM's split products (nf4_gemm_f32.hip) against
+the float64 product of the same operands (the layer's own dequantized f32
+weight, which the codec tests hold to the reference bit for bit): no larger
+than that of f32 products summed in order by the f32 matrix instruction, also
+where the terms of a sum share a sign and its rounding errors add up.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from unifur_amd import quantize as Q
+
+pytestmark = pytest.mark.gpu
+
+
+def normal(device, seed, *shape, sigma=1.0):
+    g = torch.Generator(device)
+    g.manual_seed(seed)
+    return torch.randn(*shape, generator=g, device=device) * sigma
+
+
+def layer(values, striped=None):
+    lin = Q.Nf4Linear.from_values(values.contiguous(), values.shape[0], values.shape[1], striped=striped)
+    return lin, lin.dequantized_weight().view(values.shape).double()
+
+
+def rel(y, ref):
+    return float((y.double() - ref).norm() / ref.norm())
+
+
+# 512 rows x 8320 outputs are 260 tiles: one slab over all of the reduction,
+# the longest chain of additions.  The bounds are what the f32 instruction
+# shows at these shapes for operands of one sign.
+ONE_SIGN = {4096: 8.8e-7, 11008: 1.45e-6, 11000: 1.45e-6}
+
+
+@pytest.mark.parametrize("shift", [False, True])
+@pytest.mark.parametrize("K", [4096, 11008])
+def test_sums_of_one_sign_forward(device, K, shift):
+    w, x = normal(device, 1, K, 8320, sigma=0.02), normal(device, 2, 512, K)
+    lin, wd = layer(w + 0.005 if shift else w.abs())
+    x = x + 1.0 if shift else x.abs()
+    assert rel(lin.forward(x), x.double() @ wd) <= ONE_SIGN[K]
+
+
+@pytest.mark.parametrize("N", [4096, 11008])
+def test_sums_of_one_sign_dx(device, N):
+    lin, wd = layer(normal(device, 3, 8320, N, sigma=0.02).abs())
+    dy = normal(device, 4, 512, N, sigma=1e-3).abs()
+    assert rel(lin.backward(dy), dy.double() @ wd.t()) <= ONE_SIGN[N]
+
+
+def test_sums_of_one_sign_bf16_activations(device):
+    K = 11000  # no multiple of 64: the f32 GEMM with bf16 activations
+    lin, wd = layer(normal(device, 5, K, 8320, sigma=0.02).abs())
+    x = normal(device, 6, 512, K).abs().bfloat16()
+    assert rel(lin.forward(x, out_dtype=torch.float32), x.double() @ wd) <= ONE_SIGN[K]
+
+
+def test_sums_of_one_sign_in_turn(device):
+    """The slabs taken in turn (no room for partials) to the same bits."""
+    K, N = 11008, 2048
+    lin, wd = layer(normal(device, 7, K, N, sigma=0.02).abs())
+    x = normal(device, 8, 300, K).abs()
+    y = lin.forward(x)
+    assert rel(y, x.double() @ wd) <= ONE_SIGN[K]

@@ -14,24 +14,32 @@
 // Products.  Each f32 operand is cut into three bf16 terms by truncation,
 // v = hi + mid + lo exactly (8 + 8 + 8 significand bits; no rounding, so no
 // term overflows), and the product is the six bf16 products whose terms reach
-// 2^-16 of it (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi), accumulated in
-// f32 by v_mfma_f32_32x32x16_bf16; what is left out is under 2^-23 of a
-// product.  Six of these take 192 matrix-core cycles per 32 x 32 x 16 where
-// v_mfma_f32_32x32x2f32 takes 512, and round the accumulator six times
-// instead of eight.  Relative 2-norm error against float64, N(0, 1)
-// activations, before (f32 instruction, one slab) and now: d_in 64
-// 1.33e-7 and 1.30e-7, 512 3.9e-7 and 2.5e-7, 4096 1.1e-6 and 5.0e-7 (four
-// slabs) or 1.01e-6 (one).  Infinities and NaN have no such split: a wave
-// with a sum that is not finite computes its tiles again with the f32
-// instruction, from the same operands (exact_tile).  A bf16 X (XBF) is its
-// own hi term, so its products with the weight's three terms are exact and
-// there are three of them: the path of bf16 batches whose shape the bf16
-// kernels do not take, where the weight stays the exact f32 one.
+// 2^-15 of it (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi), accumulated in
+// f32 by v_mfma_f32_32x32x16_bf16; what is left out is under 2^-21 of a
+// product.  hi hi has an accumulator of its own, the other five share a
+// second, and the two are added once at the end: added to the sum of hi hi,
+// the small products would fall below half a unit of it once it is large and
+// be lost, towards zero.  Six of these take 192 matrix-core cycles per
+// 32 x 32 x 16 where v_mfma_f32_32x32x2f32 takes 512, and round the large
+// accumulator once instead of eight times.  Relative 2-norm error against
+// float64, 512 rows -> 8320 (one slab), of the f32 instruction, of six
+// products in one accumulator, and now: N(0, 1) activations, d_in 4096
+// 1.09e-6, 1.01e-6, 3.8e-7, d_in 11008 1.79e-6, 1.75e-6, 6.5e-7; operands of
+// one sign, 8.9e-7, 9.6e-6, 3.4e-7 and 1.46e-6, 1.76e-5, 5.4e-7.  Infinities
+// and NaN have no such split: a wave with a sum that is not finite computes
+// its tiles again with the f32 instruction, from the same operands
+// (exact_tile).  A bf16 X (XBF) is its own hi term, so its products with the
+// weight's three terms are exact and there are three of them: the path of bf16
+// batches whose shape the bf16 kernels do not take, where the weight stays
+// the exact f32 one.
 //
-// What bounds it: the matrix cores' power.  2048 x 4096 -> 4096 in 373 us
+// What bounds it: the matrix cores' power.  2048 x 4096 -> 4096 in 363 us
 // (601 with the f32 instruction) is 1.1 PFLOP/s of bf16 products, what a
-// large bf16 product reaches here; 500 rows 118 us and a reduction of 7
-// (366 before, when 128 tiles left half the CUs idle; now four slabs of K).
+// large bf16 product reaches here; 500 rows 108 us with the reduction (366
+// before, when 128 tiles left half the CUs idle; now four slabs of K).  The
+// second accumulator costs registers (134 -> 206 at 128 rows): two workgroups
+// a CU, no third where a grid has more than two a CU (1024 x 4096 -> 11008
+// 594 -> 624 us; 2048 x 4096 -> 4096 369 -> 363, 500 rows 109 -> 108).
 //
 // Tiling.  A 256-thread workgroup owns 32 RT rows x 128 columns, K in steps
 // of 32; each of its four waves owns 32 columns of all the rows, so that a
@@ -251,8 +259,9 @@ __device__ __forceinline__ void slab_sums(f32x16 (&acc)[RT], const F32GemmArgs& 
   store_x<RT, XBF>(x, 0, tid);
   __syncthreads();  // X of the first step, and the LUTs
 
+  f32x16 low[RT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) acc[i] = f32x16{};
+  for (int i = 0; i < RT; ++i) acc[i] = low[i] = f32x16{};
   const uint32_t stage = (uint32_t)(S::kCodes + wave * 512 + lane * 8);
   int buf = 0;
   for (int k0 = kb; k0 < ke; k0 += kFK, buf ^= 1) {
@@ -288,18 +297,18 @@ __device__ __forceinline__ void slab_sums(f32x16 (&acc)[RT], const F32GemmArgs& 
 #pragma unroll
         for (int q = 0; q < (XBF ? 1 : 3); ++q)
           xp[q] = *reinterpret_cast<lds_u32x4*>((size_t)x_at(buf * S::kBuf + q * S::kPlane, 32 * i + r32, 2 * h + d));
-        const auto mul = [&](int a, int c) {
-          acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xp[a]),
-                                                           __builtin_bit_cast(bf16x8_t, wp[c]), acc[i], 0, 0, 0);
+        const auto mul = [&](f32x16& sum, int a, int c) {
+          sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xp[a]),
+                                                        __builtin_bit_cast(bf16x8_t, wp[c]), sum, 0, 0, 0);
         };
-        if constexpr (!XBF) mul(2, 0);
-        mul(0, 2);
+        mul(acc[i], 0, 0);
+        if constexpr (!XBF) mul(low[i], 2, 0);
+        mul(low[i], 0, 2);
         if constexpr (!XBF) {
-          mul(1, 1);
-          mul(1, 0);
+          mul(low[i], 1, 1);
+          mul(low[i], 1, 0);
         }
-        mul(0, 1);
-        mul(0, 0);
+        mul(low[i], 0, 1);
       }
     }
     c0 = c1;
@@ -308,6 +317,10 @@ __device__ __forceinline__ void slab_sums(f32x16 (&acc)[RT], const F32GemmArgs& 
     __syncthreads();
   }
 
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] += low[i][r];
   // a sum that is not finite: the wave's tiles again, with the f32
   // instruction (the wave as one: an MFMA reads every lane's operands)
   bool finite = true;
@@ -338,9 +351,11 @@ __device__ __forceinline__ void slab_sums(f32x16 (&acc)[RT], const F32GemmArgs& 
 
 // One workgroup a (tile, slab), or with SERIAL one a tile that takes the
 // slabs in turn and adds their sums in the order of the reduction: a call
-// gives the same bits with and without room for the partials.
+// gives the same bits with and without room for the partials.  SERIAL has at
+// most 256 workgroups (two slabs or more of kF32Grid), so one a CU is enough
+// and its third set of sums stays in registers.
 template <int RT, bool DQ, bool STRIPED, bool TRANS, bool XBF, bool SERIAL>
-__global__ __launch_bounds__(kFThreads, 2) void gemm_f32_kernel(F32GemmArgs g) {
+__global__ __launch_bounds__(kFThreads, SERIAL && RT == 4 ? 1 : 2) void gemm_f32_kernel(F32GemmArgs g) {
   using S = FSmem<RT>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
