@@ -65,3 +65,22 @@ def test_sums_of_one_sign_in_turn(device):
     x = normal(device, 8, 300, K).abs()
     y = lin.forward(x)
     assert rel(y, x.double() @ wd) <= ONE_SIGN[K]
+
+
+@pytest.mark.parametrize("dq", [True, False])
+@pytest.mark.parametrize("striped", [True, False])
+def test_rows_of_the_identity_give_the_dequantized_weight(device, striped, dq):
+    """One exact product a sum: the weight operand is the f32 value of the
+    format (level * scale, rounded once), bit for bit."""
+    K, N = 320, 448
+    p = Q.PackedNf4Tensor.quantize(normal(device, 9, K * N, sigma=0.02))
+    lin = Q.Nf4Linear.from_packed(p.with_double_quantization() if dq else p, K, N, striped=striped)
+    w = lin.dequantized_weight().view(K, N)
+    assert torch.equal(lin.forward(torch.eye(K, device=device)), w)
+    assert torch.equal(lin.backward(torch.eye(N, device=device)), w.t())
+    # d_in no multiple of 64: the same kernel with bf16 activations
+    K = 328
+    p = Q.PackedNf4Tensor.quantize(normal(device, 10, K * N, sigma=0.02))
+    lin = Q.Nf4Linear.from_packed(p.with_double_quantization() if dq else p, K, N, striped=striped)
+    y = lin.forward(torch.eye(K, device=device, dtype=torch.bfloat16), out_dtype=torch.float32)
+    assert torch.equal(y, lin.dequantized_weight().view(K, N))

@@ -84,8 +84,11 @@ struct FSmem {
 __device__ __forceinline__ uint32_t fbits(float v) { return __float_as_uint(v); }
 
 // Two values' truncated bf16 terms as one dword (a in the low half), and what
-// is left of each.
+// is left of each.  No contraction: fused with the product level * scale that
+// a weight value comes from, the subtraction would leave the rest of the
+// unrounded product, and the terms would not be those of the f32 value.
 __device__ __forceinline__ uint32_t cut_pair(float& a, float& b) {
+#pragma clang fp contract(off)
   const uint32_t pk = perm_b32(fbits(b), fbits(a), 0x07060302u);
   a -= __uint_as_float(fbits(a) & 0xffff0000u);
   b -= __uint_as_float(fbits(b) & 0xffff0000u);
