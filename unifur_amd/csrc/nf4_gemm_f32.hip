@@ -11,27 +11,31 @@
 // of the same function with the base weight frozen (src/qwentrain.rs:421-470).
 // No weight-sized scratch: each workgroup dequantizes the W tiles it needs.
 //
-// Products.  Each f32 operand is cut into three bf16 terms by truncation,
-// v = hi + mid + lo exactly (8 + 8 + 8 significand bits; no rounding, so no
-// term overflows), and the product is the six bf16 products whose terms reach
-// 2^-15 of it (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi), accumulated in
-// f32 by v_mfma_f32_32x32x16_bf16; what is left out is under 2^-21 of a
-// product.  hi hi has an accumulator of its own, the other five share a
-// second, and the two are added once at the end: added to the sum of hi hi,
-// the small products would fall below half a unit of it once it is large and
-// be lost, towards zero.  Six of these take 192 matrix-core cycles per
-// 32 x 32 x 16 where v_mfma_f32_32x32x2f32 takes 512, and round the large
-// accumulator once instead of eight times.  Relative 2-norm error against
-// float64, 512 rows -> 8320 (one slab), of the f32 instruction, of six
-// products in one accumulator, and now: N(0, 1) activations, d_in 4096
-// 1.09e-6, 1.01e-6, 3.8e-7, d_in 11008 1.79e-6, 1.75e-6, 6.5e-7; operands of
-// one sign, 8.9e-7, 9.6e-6, 3.4e-7 and 1.46e-6, 1.76e-5, 5.4e-7.  Infinities
-// and NaN have no such split: a wave with a sum that is not finite computes
-// its tiles again with the f32 instruction, from the same operands
-// (exact_tile).  A bf16 X (XBF) is its own hi term, so its products with the
-// weight's three terms are exact and there are three of them: the path of bf16
-// batches whose shape the bf16 kernels do not take, where the weight stays
-// the exact f32 one.
+// Products.  Each f32 operand is cut into three bf16 terms, each the nearest
+// to what the ones before leave, v = hi + mid + lo exactly, and the product is
+// six bf16 products (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi),
+// accumulated in f32 by v_mfma_f32_32x32x16_bf16.  mid is at most 2^-8 and lo
+// 2^-17 of a value's power of two, so that what is left out is under 2^-24 of
+// a product, 0.6e-8 rms, of either sign (terms cut by truncation leave 2^-21,
+// always of the product's sign).  hi hi has an accumulator of its own, the
+// other five share a second, and the two are added once at the end: added to
+// the sum of hi hi, the small products would fall below half a unit of it once
+// it is large and be lost, towards zero.  Six of these take 192 matrix-core
+// cycles per 32 x 32 x 16 where v_mfma_f32_32x32x2f32 takes 512, and round the
+// large accumulator once instead of eight times.  Relative 2-norm error
+// against float64, 512 rows -> 8320 (one slab), of the f32 instruction and
+// now, for N(0, 1) activations and for operands of one sign:
+//   d_in 4      3.9e-8 2.6e-8   3.5e-8 2.6e-8
+//   d_in 64     1.4e-7 4.3e-8   1.1e-7 4.5e-8
+//   d_in 4096   1.1e-6 3.7e-7   8.9e-7 3.3e-7
+//   d_in 11008  1.8e-6 6.5e-7   1.5e-6 5.4e-7
+// (one product a sum: 2.53e-8 and 2.59e-8, at most 2^-24 and 2^-23.3).
+// Infinities and NaN, and a value that rounds to an infinity, have no such
+// split: a wave with a sum that is not finite computes its tiles again with
+// the f32 instruction, from the same operands (exact_tile).  A bf16 X (XBF) is
+// its own hi term, so its products with the weight's three terms are exact and
+// there are three of them: the path of bf16 batches whose shape the bf16
+// kernels do not take, where the weight stays the exact f32 one.
 //
 // What bounds it: the matrix cores' power.  2048 x 4096 -> 4096 in 363 us
 // (601 with the f32 instruction) is 1.1 PFLOP/s of bf16 products, what a
@@ -83,19 +87,21 @@ struct FSmem {
 
 __device__ __forceinline__ uint32_t fbits(float v) { return __float_as_uint(v); }
 
-// Two values' truncated bf16 terms as one dword (a in the low half), and what
-// is left of each.  No contraction: fused with the product level * scale that
-// a weight value comes from, the subtraction would leave the rest of the
-// unrounded product, and the terms would not be those of the f32 value.
+// Two values' bf16 terms, rounded to nearest, as one dword (a in the low
+// half), and what is left of each (exact: at most half the term's last place).
+// No contraction: fused with the product level * scale that a weight value
+// comes from, the subtraction would leave the rest of the unrounded product,
+// and the terms would not be those of the f32 value.
 __device__ __forceinline__ uint32_t cut_pair(float& a, float& b) {
 #pragma clang fp contract(off)
-  const uint32_t pk = perm_b32(fbits(b), fbits(a), 0x07060302u);
-  a -= __uint_as_float(fbits(a) & 0xffff0000u);
-  b -= __uint_as_float(fbits(b) & 0xffff0000u);
+  const uint32_t pk = pack_bf16x2(a, b);
+  a -= bf16_bits_to_f32(pk);
+  b -= __uint_as_float(pk & 0xffff0000u);
   return pk;
 }
 
-// Eight values -> their hi, mid and lo planes, eight bf16 each.
+// Eight values -> their hi, mid and lo planes, eight bf16 each (what is left
+// after two terms has at most eight significant bits).
 __device__ __forceinline__ void split8(float (&v)[8], u32x4 (&p)[3]) {
 #pragma unroll
   for (int q = 0; q < 2; ++q)
