@@ -57,8 +57,8 @@ def test_forward(device, oracle, shape, striped):
 @pytest.mark.parametrize("scale", [1e-30, 1e30, 3.0e38])
 def test_magnitudes(device, oracle, scale):
     """The largest f32 values round to an infinite first term, which leads to
-    the f32 instruction; at 1e-30 the smallest term is still a normal bf16
-    number."""
+    the f32 instruction, and so do values that the scaling before the cut
+    takes past it."""
     M, K, N = 96, 512, 128
     lin, wdeq = make_linear(oracle, K, N, 0xB4, device)
     x, _ = acts(oracle, M, K, 0xB5, torch.float32, device)

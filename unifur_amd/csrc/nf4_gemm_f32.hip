@@ -30,20 +30,24 @@
 //   d_in 4096   1.1e-6 3.7e-7   8.9e-7 3.3e-7
 //   d_in 11008  1.8e-6 6.5e-7   1.5e-6 5.4e-7
 // (one product a sum: 2.53e-8 and 2.59e-8, at most 2^-24 and 2^-23.3).
-// Infinities and NaN, and a value that rounds to an infinity, have no such
-// split: a wave with a sum that is not finite computes its tiles again with
-// the f32 instruction, from the same operands (exact_tile).  A bf16 X (XBF) is
+// A value's terms are bf16 numbers down to the subnormals because X is cut
+// at 2^24 times its size (kXScale).  Infinities and NaN, a scaled value or sum
+// past the largest f32 and weights of the smallest scales have no such split:
+// a wave with a sum that is not finite computes its tiles again with the f32
+// instruction, from the same operands (exact_tile).  A bf16 X (XBF) is
 // its own hi term, so its products with the weight's three terms are exact and
 // there are three of them: the path of bf16 batches whose shape the bf16
 // kernels do not take, where the weight stays the exact f32 one.
 //
-// What bounds it: the matrix cores' power.  2048 x 4096 -> 4096 in 363 us
-// (601 with the f32 instruction) is 1.1 PFLOP/s of bf16 products, what a
-// large bf16 product reaches here; 500 rows 108 us with the reduction (366
-// before, when 128 tiles left half the CUs idle; now four slabs of K).  The
-// second accumulator costs registers (134 -> 206 at 128 rows): two workgroups
-// a CU, no third where a grid has more than two a CU (1024 x 4096 -> 11008
-// 594 -> 624 us; 2048 x 4096 -> 4096 369 -> 363, 500 rows 109 -> 108).
+// What bounds it: at 2048 x 4096 -> 4096, 370 us (601 with the f32
+// instruction), the matrix cores' power: 1.1 PFLOP/s of bf16 products, what a
+// large bf16 product reaches here.  500 rows take 110 us (366 with the f32
+// instruction, whose 128 tiles left half the CUs idle; now four slabs of K):
+// 0.9 PFLOP/s, the rest being the slabs' partials, 33 MB written and read, the
+// reduction launch, and the weight decoded and cut once per 128 rows.  The
+// second accumulator costs registers (134 -> 205 at 128 rows, two workgroups a
+// CU) but no time: 2048 rows 380 us with one and 370 with two, 500 rows 112
+// and 110, 1024 x 4096 -> 11008 606 and 577, 64 x 4096 -> 11008 52 and 51.
 //
 // Tiling.  A 256-thread workgroup owns 32 RT rows x 128 columns, K in steps
 // of 32; each of its four waves owns 32 columns of all the rows, so that a
@@ -85,7 +89,22 @@ struct FSmem {
   static constexpr int kBytes = kDq + 256 * 4;
 };
 
+// The terms of every f32 value have to be bf16 numbers.  A bf16 number has no
+// bits below 2^-133, and an f32 value under 2^-110 has some, so X is
+// multiplied by 2^24 before it is cut (exact; the sums are divided by it
+// again, and one that overflows for it is not finite: exact_tile).  A weight
+// value's scale under 2^-99, whose terms could be as small, is taken as NaN,
+// which leads there too.
+constexpr float kXScale = 16777216.0f;
+constexpr uint32_t kTinyScale = (127u - 99u) << 23;
+
 __device__ __forceinline__ uint32_t fbits(float v) { return __float_as_uint(v); }
+
+__device__ __forceinline__ float dq_scale(int q, float scale_of_scales) { return ((float)q / 255.0f) * scale_of_scales; }
+
+__device__ __forceinline__ float no_tiny_scale(float s) {
+  return (fbits(s) & 0x7fffffffu) - 1u < kTinyScale - 1u ? __uint_as_float(0x7fc00000u) : s;
+}
 
 // Two values' bf16 terms, rounded to nearest, as one dword (a in the low
 // half), and what is left of each (exact: at most half the term's last place).
@@ -160,6 +179,7 @@ __device__ __forceinline__ FCodes load_codes(const F32GemmArgs& g, const FLane<S
 }
 
 // The X values of a step this thread stages: 4 RT consecutive k of one row.
+// Past the end of the row its last ones again: they meet weights of zero.
 template <int RT, bool XBF>
 struct FX {
   f32x4 v[XBF ? RT / 2 : RT];  // XBF: eight bf16 each
@@ -167,25 +187,14 @@ struct FX {
 
 template <int RT, bool XBF>
 __device__ __forceinline__ FX<RT, XBF> load_x(const F32GemmArgs& g, int m0, int k0, int tid) {
-  constexpr int kPerRow = 8 / RT;  // threads a row
+  constexpr int kPerRow = 8 / RT, kRun = XBF ? 8 : 4;  // threads a row; k of a load (K is a multiple)
   FX<RT, XBF> x;
   const size_t at = (size_t)min(m0 + tid / kPerRow, g.M - 1) * g.K;
-  if constexpr (XBF) {
-    const uint16_t* row = static_cast<const uint16_t*>(g.x) + at;
 #pragma unroll
-    for (int q = 0; q < RT / 2; ++q) {
-      const int k = k0 + 4 * RT * (tid % kPerRow) + 8 * q;  // K % 8 == 0
-      const f32x4 v = *reinterpret_cast<const f32x4*>(row + min(k, g.K - 8));
-      x.v[q] = k < g.K ? v : f32x4{};
-    }
-    return x;
-  }
-  const float* row = static_cast<const float*>(g.x) + at;
-#pragma unroll
-  for (int q = 0; q < (XBF ? 0 : RT); ++q) {
-    const int k = k0 + 4 * RT * (tid % kPerRow) + 4 * q;  // K % 4 == 0: a run is inside or outside a row
-    const f32x4 v = *reinterpret_cast<const f32x4*>(row + min(k, g.K - 4));
-    x.v[q] = k < g.K ? v : f32x4{};
+  for (int q = 0; q < 4 * RT / kRun; ++q) {
+    const size_t i = at + min(k0 + 4 * RT * (tid % kPerRow) + kRun * q, g.K - kRun);
+    x.v[q] = XBF ? *reinterpret_cast<const f32x4*>(static_cast<const uint16_t*>(g.x) + i)
+                 : *reinterpret_cast<const f32x4*>(static_cast<const float*>(g.x) + i);
   }
   return x;
 }
@@ -211,6 +220,8 @@ __device__ __forceinline__ void store_x(const FX<RT, XBF>& x, int buf, int tid) 
     for (int c = 0; c < RT / 2; ++c) {
       float v[8] = {x.v[2 * c].x,     x.v[2 * c].y,     x.v[2 * c].z,     x.v[2 * c].w,
                     x.v[2 * c + 1].x, x.v[2 * c + 1].y, x.v[2 * c + 1].z, x.v[2 * c + 1].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= kXScale;
       u32x4 p[3];
       split8(v, p);
 #pragma unroll
@@ -226,7 +237,7 @@ template <int RT, bool DQ, bool STRIPED, bool TRANS, bool XBF>
 __device__ void exact_tile(f32x16 (&acc)[RT], const F32GemmArgs& g, const unsigned char* smem, int m0, int n, int kb,
                            int ke, int lane) {
   const float* lut = reinterpret_cast<const float*>(smem + FSmem<RT>::kLut);  // lut[2 c] = level c, c < 16
-  const float* dq_lut = reinterpret_cast<const float*>(smem + FSmem<RT>::kDq);
+  const float sos = DQ ? *g.scales.scale_of_scales : 0.0f;
 #pragma unroll
   for (int i = 0; i < RT; ++i) acc[i] = f32x16{};
   const int nn = min(n, g.N - 1);
@@ -240,7 +251,7 @@ __device__ void exact_tile(f32x16 (&acc)[RT], const F32GemmArgs& g, const unsign
         STRIPED ? ((size_t)(wc / 16) * wrows + wr) * 8 + (wc & 15) / 2 : (size_t)wr * (wcols / 2) + wc / 2;
     const size_t blk = STRIPED ? (size_t)(wc / kBlock) * wrows + wr : (size_t)wr * (wcols / kBlock) + wc / kBlock;
     const int code = (g.packed[at] >> (4 * (wc & 1))) & 15;
-    const float s = DQ ? dq_lut[g.scales.dq_codes[blk]] : g.scales.absmax[blk];
+    const float s = DQ ? dq_scale(g.scales.dq_codes[blk], sos) : g.scales.absmax[blk];
     const float w = in ? lut[2 * code] * s : 0.0f;
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
@@ -285,6 +296,7 @@ __device__ __forceinline__ void slab_sums(f32x16 (&acc)[RT], const F32GemmArgs& 
       nib = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr4_b64_v2i32(reinterpret_cast<lds_v2i32*>((size_t)stage)));
     }
     float s = DQ ? dq_lut[c0.scale & 0xffu] : __uint_as_float(c0.scale);
+    if constexpr (!DQ) s = no_tiny_scale(s);
     s = c0.live ? s : 0.0f;
     float sc[16];
     if constexpr (!TRANS) row_lanes<0>(s, sc);  // row 16 h + j's scale sits in lane 16 (l / 16) + j
@@ -337,8 +349,12 @@ __device__ __forceinline__ void slab_sums(f32x16 (&acc)[RT], const F32GemmArgs& 
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) finite = finite && (fbits(acc[i][r]) & 0x7f800000u) != 0x7f800000u;
-  if (__any(!finite))
+  if (__any(!finite)) {
     exact_tile<RT, DQ, STRIPED, TRANS, XBF>(acc, g, smem, m0, n0 + r32, kb, ke, lane);
+  } else if constexpr (!XBF) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) acc[i] *= 1.0f / kXScale;
+  }
 
   // the adapter, in the first slab's sums: acc += (xa scaling) B over the
   // rank; xa [M][lora_ld] f32 and B element (j, n) at lora_b[j sbj + n sbn]
@@ -383,7 +399,7 @@ __global__ __launch_bounds__(kFThreads, SERIAL && RT == 4 ? 1 : 2) void gemm_f32
     lut[2 * tid] = level(tid & 15);
     lut[2 * tid + 1] = level(tid >> 4);
     if constexpr (DQ)
-      reinterpret_cast<float*>(smem + S::kDq)[tid] = ((float)tid / 255.0f) * (*g.scales.scale_of_scales);
+      reinterpret_cast<float*>(smem + S::kDq)[tid] = no_tiny_scale(dq_scale(tid, *g.scales.scale_of_scales));
     __syncthreads();
   }
   f32x16 acc[RT];
