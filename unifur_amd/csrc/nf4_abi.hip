@@ -125,7 +125,8 @@ WsCache& ws_cache() {
 // find it alive.  Under stream capture nothing is allocated, synchronized or
 // filled: a call that would have to create or grow the buffer there fails
 // with UNIFUR_NF4_ERR_WORKSPACE (make one eager call of the largest shape
-// first, or pass a workspace).
+// first, or pass a workspace); see workspace_holds for the one plan that then
+// goes on with less.
 int internal_workspace(size_t bytes, hipStream_t stream, void** out) {
   int dev = 0;
   UNIFUR_HIP(hipGetDevice(&dev));
@@ -174,11 +175,16 @@ int resolve_workspace(void* user, uint64_t user_bytes, size_t need, hipStream_t 
 
 // Whether a call's workspace can hold `need` bytes: the caller's as it is,
 // the internal one after growing to them (not under capture, nor when the
-// device is out of memory).  For plans that have a leaner form.
+// device is out of memory).  For the f32 GEMM's slab partials, without which
+// its call gives the same bits: the only plan whose internal workspace may
+// turn out smaller (every other one is refused under capture, so that a graph
+// never holds a slower form unnoticed).  Leaves no error text behind.
 bool workspace_holds(void* user, uint64_t user_bytes, size_t need, hipStream_t stream) {
   if (user) return user_bytes >= need;
+  const std::string text = g_last_error;
   void* p = nullptr;
   if (internal_workspace(need, stream, &p) == UNIFUR_NF4_OK) return true;
+  g_last_error = text;
   (void)hipGetLastError();  // a failed allocation's error
   return false;
 }
@@ -446,7 +452,7 @@ int run_linear(const void* x, int x_dtype, uint64_t rows, const unifur_nf4_weigh
                                allow_expand);
   if (L.path == LinearPath::kMid) {
     if (L.gemm_partials && (!aligned_to(y, 16) || !aligned_to(bias, 16) ||
-                            !workspace_holds(workspace, workspace_bytes, L.total, stream))) {
+                            (workspace && workspace_bytes < L.total))) {
       L.gemm_partials = 0;
       L.total = L.lean;
     }
@@ -477,9 +483,11 @@ int run_linear(const void* x, int x_dtype, uint64_t rows, const unifur_nf4_weigh
                                                 std::to_string(lean.total) + " bytes of workspace here, got " +
                                                 std::to_string(workspace_bytes));
   }
-  if (((L.path == LinearPath::kMfma && !L.expand && (L.splits > 1 || L.tail > 1)) ||
-       (L.path == LinearPath::kMfmaF32 && L.splits > 1)) &&
-      (!aligned_to(y, 16) || !aligned_to(bias, 16) || !workspace_holds(workspace, workspace_bytes, L.total, stream))) {
+  const bool split_mfma = L.path == LinearPath::kMfma && !L.expand && (L.splits > 1 || L.tail > 1);
+  const bool split_f32 = L.path == LinearPath::kMfmaF32 && L.splits > 1;
+  if ((split_mfma || split_f32) &&
+      (!aligned_to(y, 16) || !aligned_to(bias, 16) || (workspace && workspace_bytes < L.total) ||
+       (split_f32 && !workspace_holds(workspace, workspace_bytes, L.total, stream)))) {
     // no room for the split-K partials (or an output or bias the reduction
     // cannot access four at a time): the fused kernel over whole d_in
     L = plan_linear(rows, w->d_in, w->d_out, rank, w->packed, x_dtype, x, is_striped(w), w->scales.kind, false,
@@ -790,7 +798,8 @@ int run_swiglu(const void* x, int x_dtype, uint64_t rows, const unifur_nf4_weigh
                                                 std::to_string(workspace_bytes));
   }
   if (((L.path == MlpPath::kMfma && !L.expand) || L.f32_mfma) && L.gemm_partials &&
-      (!aligned_to(y, 16) || !workspace_holds(workspace, workspace_bytes, L.total, stream)))
+      (!aligned_to(y, 16) || (workspace && workspace_bytes < L.total) ||
+       (L.f32_mfma && !workspace_holds(workspace, workspace_bytes, L.total, stream))))
     L = plan_mlp(rows, hidden, inter, gate, up, down, x_dtype, x, false, false);  // without split-K
   void* ws = nullptr;
   if (int r = resolve_workspace(workspace, workspace_bytes, L.total, stream, &ws)) return r;
@@ -1490,7 +1499,8 @@ int run_attn_in(const void* x, int dtype, uint64_t rows, const unifur_nf4_decode
     return UNIFUR_NF4_OK;
   }
   AttnInLayout L = plan_attn_in(rows, l, dtype);
-  if (!workspace_holds(workspace, workspace_bytes, L.total, stream))  // without the linears' split-K partials
+  // f32: without the linears' slab partials where there is no room for them
+  if (dtype == UNIFUR_NF4_F32 && !workspace_holds(workspace, workspace_bytes, L.total, stream))
     L = plan_attn_in(rows, l, dtype, false);
   void* ws = nullptr;
   if (int r = resolve_workspace(workspace, workspace_bytes, L.total, stream, &ws)) return r;
@@ -1590,7 +1600,8 @@ int run_attn_out_mlp(const void* x, const void* ctx, int dtype, uint64_t rows, c
   const bool bf = dtype == UNIFUR_NF4_BF16;
   const uint64_t hid = l->o.d_out, inter = l->gate.d_out;
   AttnOutLayout L = plan_attn_out(rows, l, dtype, ctx, reinterpret_cast<const void*>(uintptr_t{256}));
-  if (!workspace_holds(workspace, workspace_bytes, L.total, stream))  // without the linears' split-K partials
+  // f32: without the linears' slab partials where there is no room for them
+  if (!bf && !workspace_holds(workspace, workspace_bytes, L.total, stream))
     L = plan_attn_out(rows, l, dtype, ctx, reinterpret_cast<const void*>(uintptr_t{256}), false);
   void* ws = nullptr;
   if (int r = resolve_workspace(workspace, workspace_bytes, L.total, stream, &ws)) return r;
