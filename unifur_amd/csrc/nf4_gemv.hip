@@ -204,8 +204,11 @@ __device__ __forceinline__ void accumulate(float (&acc)[T][32], const RowLoads<R
   }
 }
 
+// bias and adapter; a pair launch (PAIR) has neither
+template <bool PAIR>
 __device__ __forceinline__ float epilogue_value(const GemvWeight& W, float base, int t, int gcol) {
   float y = base;
+  if constexpr (PAIR) return y;
   if (W.bias) y += W.bias[gcol];
   if (W.lora_xa) {
     // base(x) + ((x A) B) * scaling (src/qwennet.rs:325-344, src/quantize.rs:619-624)
@@ -350,8 +353,8 @@ __global__ __launch_bounds__(kThreads) void gemv_splitk_kernel(GemvArgs a) {
   if (!gcol_ok) return;
 #pragma unroll
   for (int t = 0; t < T; ++t) {
-    float y = epilogue_value(W, res0[t], t, gcol);
-    if constexpr (PAIR) y = silu_f32(y) * epilogue_value(a.w[1], res1[t], t, gcol);  // silu(gate x) * up x
+    float y = epilogue_value<PAIR>(W, res0[t], t, gcol);
+    if constexpr (PAIR) y = silu_f32(y) * epilogue_value<PAIR>(a.w[1], res1[t], t, gcol);  // silu(gate x) * up x
     store_y(W, (size_t)t * N + gcol, y);
   }
 }
@@ -446,6 +449,7 @@ GemvPlan plan_gemv(int rows, int d_in, const int* d_out, int nweights, bool pair
 
 hipError_t launch_gemv(const GemvPlan& p, const void* x, bool x_bf16, int rows, int d_in, const GemvWeight* weights,
                        int nweights, hipStream_t stream) {
+  if (p.pair && !pair_weights_plain(weights)) return hipErrorInvalidValue;
   GemvArgs a{};
   a.x = x;
   a.rows = rows;

@@ -47,6 +47,15 @@ __device__ __forceinline__ float adapter_dot(const float* xa, const float* b, si
   return l;
 }
 
+// A pair launch (gate / up) carries neither bias nor adapter: its kernels are
+// built without them (with the adapter's loads in their epilogue the f32
+// skinny pair went from three waves a SIMD to two and the 64-row bf16 one
+// from 4 spilled registers to 9: 4096 / 11008 decoder stage, 64 rows, 101 ->
+// 105 us).
+inline bool pair_weights_plain(const GemvWeight* w) {
+  return !w[0].bias && !w[0].lora_xa && !w[1].bias && !w[1].lora_xa;
+}
+
 struct GemvPlan {
   bool pair;  // gate/up SwiGLU pair: weights[0], weights[1] share x and d_out
   int rows_per_thread;

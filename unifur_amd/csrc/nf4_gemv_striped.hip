@@ -304,8 +304,11 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// bias and adapter; a pair launch (PAIR) has neither
+template <bool PAIR>
 __device__ __forceinline__ float epilogue_value(const GemvWeight& W, float base, int t, int gcol) {
   float y = base;
+  if constexpr (PAIR) return y;
   if (W.bias) y += W.bias[gcol];
   if (W.lora_xa) {
     // base(x) + ((x A) B) * scaling (src/qwennet.rs:325-344, src/quantize.rs:619-624)
@@ -524,8 +527,8 @@ __global__ __launch_bounds__(W * 64) void gemv_striped_kernel(const void* x_arg,
 #pragma unroll
     for (int w = 0; w < NW; ++w) sum[w] *= inv;
   }
-  float y = epilogue_value(G, sum[0], t, gcol);
-  if constexpr (PAIR) y = silu_f32(y) * epilogue_value(a.w[1], sum[1], t, gcol);  // silu(gate x) * up x
+  float y = epilogue_value<PAIR>(G, sum[0], t, gcol);
+  if constexpr (PAIR) y = silu_f32(y) * epilogue_value<PAIR>(a.w[1], sum[1], t, gcol);  // silu(gate x) * up x
   store_y(G, (size_t)t * G.d_out + gcol, y);
 }
 
@@ -1055,8 +1058,8 @@ __global__ __launch_bounds__(W * 64) void skinny_kernel(const void* x_arg, const
 #pragma unroll
     for (int i = 0; i < S; ++i) {
       const int gcol = (s0 + i) * kStripeCols + cc;
-      float y = epilogue_value(G, sums[0][i][tt] * nrm, t, gcol);
-      if constexpr (PAIR) y = silu_f32(y) * epilogue_value(a.w[1], sums[1][i][tt] * nrm, t, gcol);
+      float y = epilogue_value<PAIR>(G, sums[0][i][tt] * nrm, t, gcol);
+      if constexpr (PAIR) y = silu_f32(y) * epilogue_value<PAIR>(a.w[1], sums[1][i][tt] * nrm, t, gcol);
       store_y(G, (size_t)t * G.d_out + gcol, y);
     }
   }
@@ -1152,6 +1155,7 @@ StripedPlan plan_gemv_striped(int rows, int d_in, const int* d_out, int nweights
 hipError_t launch_gemv_striped(const StripedPlan& p, const void* x, bool x_bf16, int rows, int d_in,
                                const GemvWeight* weights, int nweights, bool pair, hipStream_t stream,
                                const float* norm_w, float norm_eps) {
+  if (pair && !pair_weights_plain(weights)) return hipErrorInvalidValue;
   StripedArgs a{};
   a.x = x;
   a.norm_w = norm_w;
@@ -1249,7 +1253,7 @@ StripedPlan plan_skinny(int rows, int d_in, const int* d_out, int nweights, bool
 hipError_t launch_skinny(const StripedPlan& p, const void* x, bool x_f32, int rows, int d_in,
                          const GemvWeight* weights, int nweights, bool pair, hipStream_t stream, const float* norm_w,
                          float norm_eps) {
-  if (!skinny_supported(rows, d_in, x, x_f32) || nweights < 1 || nweights > kMaxGemvWeights || (pair && nweights != 2))
+  if (!skinny_supported(rows, d_in, x, x_f32) || nweights < 1 || nweights > kMaxGemvWeights || (pair && (nweights != 2 || !pair_weights_plain(weights))))
     return hipErrorInvalidValue;
   if ((p.group != 1 && p.group != 2 && p.group != 4) || p.splits < 1 || p.splits > 65535 ||
       (long)p.rows_per_split * p.splits < d_in || p.rows_per_split != p.rows_per_wave * p.waves)
