@@ -16,8 +16,8 @@ import torch
 from unifur_amd import _lib as L
 from unifur_amd import quantize as Q
 
-from test_gpu_gemm import lora_parts
-from test_gpu_linear import TOL_BF16, acts, check, make_linear
+from test_gpu_gemm import lora_parts, zero_linear
+from test_gpu_linear import TOL_BF16, TOL_F32, acts, check, make_linear
 
 pytestmark = pytest.mark.gpu
 
@@ -67,6 +67,31 @@ def test_mid_rows(device, oracle, K, N, rows, r, dq):
     forward(lin, xt, rows, ad, bt, y3, full)
     assert torch.equal(y3, y.to(torch.bfloat16))
     assert torch.isnan(buf[0]) and torch.isnan(buf[1 + rows * N:]).all()
+
+
+# x A in slabs of d_in (2^18 factor elements or more): two and four rows a
+# group with a last group that is not full, four columns a lane and one, a rank
+# whose eights the GEMM's slabs do not share evenly
+@pytest.mark.parametrize("K,N,rows,r", [(8192, 2048, 65, 32), (8192, 2048, 130, 64), (8192, 2048, 99, 33),
+                                        (8192, 2112, 191, 45), (4096, 4096, 128, 64), (8256, 4096, 255, 64)])
+def test_wide_adapters(device, oracle, K, N, rows, r):
+    lin, wdeq = make_linear(oracle, K, N, 0xC6, device)
+    x, xt = acts(oracle, rows, K, 0xC7, torch.bfloat16, device)
+    a, b, ad = lora_parts(oracle, K, N, r, 0xC8, device)
+    ref = oracle.linear_ref_f64(x, wdeq) + oracle.lora_ref_f64(x, a, b, 2.0)
+    lib = L.lib()
+    full = lib.unifur_nf4_linear_workspace_size(rows, K, N, L.BF16, r)
+    least = lib.unifur_nf4_linear_min_workspace_size(rows, K, N, L.BF16, r)
+    y = forward(lin, xt, rows, ad, None, torch.empty(rows, N, device=device), full)
+    check(y, ref, x, wdeq, TOL_BF16, f"mid {rows} x {K} -> {N} rank {r}")
+    assert torch.equal(y, forward(lin, xt, rows, ad, None, torch.empty(rows, N, device=device), least))
+    # the adapter's term alone, over a weight of zeros, is f32 throughout
+    zero = zero_linear(K, N, device, True)
+    t = forward(zero, xt, rows, ad, None, torch.empty(rows, N, device=device), full).cpu().numpy()
+    bound = (np.abs(x) @ np.abs(a)) @ np.abs(b) * 2.0
+    assert float(np.max(np.abs(t - oracle.lora_ref_f64(x, a, b, 2.0)) / bound)) <= TOL_F32
+    fresh = Q.LoraAdapter.new(Q.LoraConfig.new(K, N, r), device=device)
+    assert torch.equal(Q.QloraLinear(lin, fresh).forward(xt), lin.forward(xt))
 
 
 def test_an_adapter_of_zeros_adds_nothing(device, oracle):

@@ -240,6 +240,7 @@ struct LinearLayout {
   int tail = 1;    // ... or of only its last, partly filled round of tiles
   size_t partials, xa, lora_at, lora_bt, wt, blas, wf32, rm_codes, rm_scales, gemm_partials, total;
   size_t lean;  // kMid: the workspace without the partials
+  size_t xa_part = 0;  // kMid: the partials of x A's slabs (0: none)
   size_t xa_rows = 0;  // kMfmaF32: x A by the row products goes here (0: by the narrow kernel, to xa)
 };
 
@@ -300,10 +301,13 @@ LinearLayout plan_linear(uint64_t rows, uint64_t d_in, uint64_t d_out, uint32_t 
     L.partials = c.take(L.gemv.partial_count[0] * sizeof(float));
   } else if (mid && mfma && striped && gemm_mid_wanted((int)std::min<uint64_t>(rows, 0x7fffffffu), (int)d_in, (int)d_out) &&
              gemm_mid_supported((int)rows, (int)d_in, (int)d_out, x)) {
-    // x A, then the partials of its d_in slabs, at most the bf16 weight's
-    // bytes (without them a workgroup takes the slabs in turn)
+    // x A (with the partials of its slabs), then the partials of its own d_in
+    // slabs, at most the bf16 weight's bytes (without those a workgroup takes
+    // the slabs in turn)
     L.path = LinearPath::kMid;
     L.xa = c.take((size_t)rows * lora_rank * sizeof(float));
+    const size_t xa_part = lora_rank ? lora_xa_slab_floats((int)rows, (int)d_in, (int)lora_rank) : 0;
+    if (xa_part) L.xa_part = c.take(xa_part * sizeof(float));
     L.splits = gemm_mid_splits((int)rows, (int)d_in, (int)d_out, d_in * d_out / 2);
     L.lean = c.off;
     if (split && L.splits > 1) L.gemm_partials = c.take((size_t)L.splits * rows * d_out * sizeof(float));
@@ -501,7 +505,11 @@ int run_linear(const void* x, int x_dtype, uint64_t rows, const unifur_nf4_weigh
   if (L.path == LinearPath::kMid) {
     if (lora) {
       xa = at<float>(ws, L.xa);
-      UNIFUR_HIP(launch_lora_xa(x, true, lora->a, (int)rows, (int)w->d_in, (int)rank, xa, stream));
+      if (L.xa_part)
+        UNIFUR_HIP(launch_lora_xa_slabs(static_cast<const uint16_t*>(x), lora->a, (int)rows, (int)w->d_in, (int)rank,
+                                        xa, at<float>(ws, L.xa_part), at<unsigned>(ws, 0), stream));
+      else
+        UNIFUR_HIP(launch_lora_xa(x, true, lora->a, (int)rows, (int)w->d_in, (int)rank, xa, stream));
     }
     UNIFUR_HIP(launch_gemm_mid(static_cast<const uint16_t*>(x), w->packed, to_scales(w->scales), (int)rows,
                                (int)w->d_in, (int)w->d_out, bias, xa, lora ? lora->b : nullptr, (int)rank,

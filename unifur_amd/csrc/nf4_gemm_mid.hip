@@ -20,8 +20,8 @@
 // one a CU.
 //
 // What it is for: expanding a large weight to bf16 for a library product costs
-// the same whatever the rows, 29 us in all over 4096 x 4096 and 52 over
-// 11008 x 4096 at 100 rows; this kernel and its reduction take 19 and 26
+// the same whatever the rows, 31 us in all over 4096 x 4096 and 52 over
+// 11008 x 4096 at 100 rows; this kernel and its reduction take 18 and 24
 // (gemm_mid_wanted has the rest).
 //
 // What bounds it: one wave a SIMD issues its VALU, LDS and MFMA work one after
@@ -201,8 +201,8 @@ __device__ __forceinline__ void multiply_phase(f32x16 (&acc)[RT], const MPhase<R
                                                      __builtin_bit_cast(bf16x8_t, w), acc[i], 0, 0, 0);
 }
 
-// acc = the wave's sums over the slab [kb, ke), the adapter's term with them
-// in the first slab.  `luts`: build the tables first (the first slab of a
+// acc = the wave's sums over the slab [kb, ke), and its share of the adapter's
+// ranks.  `luts`: build the tables first (the first slab of a
 // workgroup).
 //
 // Software pipeline: a phase's table lookups and X fragments are read during
@@ -246,10 +246,12 @@ __device__ __forceinline__ void slab_sums(f32x16 (&acc)[RT], const MidArgs& g, u
   for (int i = 0; i < RT; ++i) acc[i] = f32x16{};
   // (xa scaling) B on the f32 instruction, while the first loads are in
   // flight; four steps' factors are loaded together, from clamped places
-  // and zeroed past the rank
-  if (g.lora_xa && kb == 0) {
+  // and zeroed past the rank.  Each eight ranks wait out a memory latency, so
+  // the slabs take turns at them (4096 -> 4096, rank 64, 128 rows: 44 us with
+  // all of them in the first slab, 36 with this)
+  if (g.lora_xa) {
     const float* bcol = g.lora_b + nc + r32;
-    for (int j0 = 0; j0 < g.lora_rank; j0 += 8) {
+    for (int j0 = kb / g.k_slab * 8; j0 < g.lora_rank; j0 += 8 * g.k_splits) {
       float av[4][RT], bv[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -408,17 +410,28 @@ bool gemm_mid_supported(int M, int K, int N, const void* x) {
 }
 
 // Measured against the expanded weight and the library product, us per call at
-// 65 / 128 / 192 / 256 rows, without and with a rank-16 adapter (whose x A is
-// a launch of its own here and merged into the expansion there; both take one
-// path, so that an adapter of zeros adds nothing to the bit):
-//   4096 -> 4096   15.7 20.6 22.0 25.1 against 29.1 28.7 29.6 29.2
-//                  21.5 26.5 27.8 31.3 against 28.7 29.1 29.8 29.3
-//   4096 -> 8192   20.3 25.6 31.0 33.0 against 36.5 38.1 41.6 43.2
-//                  27.3 33.0 38.4 43.0 against 40.8 42.5 46.2 49.3
-//   11008 -> 4096  23.3 26.8 35.0 40.0 against 50.7 52.7 56.3 58.4
-//   4096 -> 2048   15.2 19.3 17.5 20.6 against 22.8 23.0 25.8 25.3
-//                  21.4 25.5 24.5 27.1 against 22.6 22.8 25.3 24.8
-// so from 2^24 weights up to 192 rows, from 2^25 up to 256.
+// 65 / 128 / 192 / 256 rows, without an adapter and with one of rank 16 and 64
+// (whose x A is a launch of its own here and merged into the expansion there;
+// both take one path, so that an adapter of zeros adds nothing to the bit):
+//   4096 -> 4096       16.4 20.4 21.2       against 31.4 30.9 31.7
+//            rank 16   21.3 25.8 27.3               30.8 31.1 31.1
+//            rank 64   25.3 30.8 35.3               41.8 41.7 43.3
+//   4096 -> 8192       19.2 25.6 29.8 32.2          35.0 36.3 39.1 41.2
+//            rank 16   25.1 29.7 36.2 40.0          37.4 38.8 41.9 44.2
+//            rank 64   28.9 34.2 44.0 50.1          62.7 64.7 68.3 72.3
+//   8192 -> 2048       17.0 21.5 21.7               32.3 31.3 35.1
+//            rank 16   25.7 30.1 30.1               32.3 31.3 34.9
+//            rank 64   27.9 32.0 36.3               44.7 44.0 49.0
+//   11008 -> 4096      21.9 25.6 33.0 37.7          49.8 52.1 55.5 58.5
+//            rank 64   36.7 42.8 56.5 62.0          87.2 89.6 93.5 95.0
+//   512 -> 32768       10.5 11.9 13.9               30.3 29.6 31.5
+//            rank 64   22.7 32.2 40.7               38.1 37.9 40.5
+//   16384 -> 1024      20.1 25.5 22.8               33.1 32.1 37.4
+//            rank 16   30.4 32.9 34.4               33.0 32.1 38.3
+// so from 2^24 weights up to 192 rows, from 2^25 up to 256: the line is where
+// an adapted call still gains or breaks even.  (4096 -> 2048 without an
+// adapter would gain too, 15 to 21 us against 23 to 26, but loses with one of
+// rank 16, 24 to 27 against 23 to 26.)
 bool gemm_mid_wanted(int M, int K, int N) {
   const int64_t weights = (int64_t)K * N;
   return weights >= (int64_t)1 << 24 && M <= (weights >= (int64_t)1 << 25 ? 256 : 192);

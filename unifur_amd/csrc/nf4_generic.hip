@@ -110,15 +110,19 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const void* __restrict__ 
 // wave 64 / LPK consecutive k, so a factor load is one contiguous run per
 // wave; D steps of the wave are in flight together.  The k of a wave
 // are summed across its lanes, then the 16 waves through LDS.
+// With SLABS a workgroup takes one slab of K, blockIdx.y, and the last slab to
+// arrive at a row group adds the partials in slab order (launch_xa_slabs).
 // The form before had one thread walk all of K, one dependent load pair at a
 // time: an adapted 4096 -> 4096 linear took 956 us at 1 row and 1002 us at 64
 // (bf16, rank 16); it takes 11 and 35 us with this one (5 and 17 without the
 // adapter).
 constexpr int kXaThreads = 1024;
-template <bool XBF16, int VEC, int T>
+constexpr int kXaSlabs = 4;
+template <bool XBF16, int VEC, int T, bool SLABS>
 __global__ __launch_bounds__(kXaThreads) void lora_xa_kernel(const void* __restrict__ x, const float* __restrict__ a,
                                                              int M, int K, int rank, int lpk, size_t sk, size_t sj,
-                                                             float* __restrict__ xa) {
+                                                             float* __restrict__ xa, int kslab, float* part,
+                                                             unsigned* counters) {
   constexpr int D = T == 1 ? 16 : 8;  // steps in flight (what 128 registers hold)
   __shared__ float red[kXaThreads / 64][T][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -132,7 +136,8 @@ __global__ __launch_bounds__(kXaThreads) void lora_xa_kernel(const void* __restr
   for (int t = 0; t < T; ++t)
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[t][v] = 0.0f;
-  for (int k0 = tid / lpk; k0 < K; k0 += D * kper) {
+  const int ke = SLABS ? min(K, (int)(blockIdx.y + 1) * kslab) : K;
+  for (int k0 = (SLABS ? blockIdx.y * kslab : 0) + tid / lpk; k0 < ke; k0 += D * kper) {
     // unconditional loads from clamped places, past the end zeroed after: a
     // load under a branch would wait for the one before
     float av[D][VEC], xv[D][T];
@@ -150,7 +155,7 @@ __global__ __launch_bounds__(kXaThreads) void lora_xa_kernel(const void* __restr
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      const bool in = k0 + d * kper < K;
+      const bool in = k0 + d * kper < ke;
 #pragma unroll
       for (int v = 0; v < VEC; ++v) av[d][v] = in ? av[d][v] : 0.0f;
 #pragma unroll
@@ -169,14 +174,62 @@ __global__ __launch_bounds__(kXaThreads) void lora_xa_kernel(const void* __restr
       if (lane < lpk && live) red[wave][t][j + v] = acc[t][v];
     }
   __syncthreads();
-  for (int i = tid; i < T * rank; i += kXaThreads) {
-    const int t = i / rank, c = i % rank;
-    if (m0 + t >= M) break;
+  static_assert(T * 64 <= kXaThreads, "one value a thread");
+  const int t = tid / rank, c = tid % rank;
+  const bool mine = t < T && m0 + t < M;
+  const size_t at = (size_t)(m0 + t) * rank + c;
+  if (mine) {
     float v = red[0][t][c];
 #pragma unroll
     for (int w = 1; w < kXaThreads / 64; ++w) v += red[w][t][c];
-    xa[(size_t)(m0 + t) * rank + c] = v;
+    if constexpr (SLABS) store_coherent(part + (size_t)blockIdx.y * M * rank + at, v);
+    else xa[at] = v;
   }
+  if constexpr (SLABS) {
+    // the last slab to arrive at these rows adds all of them in slab order
+    __shared__ bool last;
+    wait_all_memory();
+    __syncthreads();
+    if (tid == 0)
+      last = __hip_atomic_fetch_add(&counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+             gridDim.y - 1;
+    __syncthreads();
+    if (!last) return;
+    if (mine) {
+      float p[kXaSlabs];
+#pragma unroll
+      for (int s = 0; s < kXaSlabs; ++s)
+        p[s] = load_coherent(part + (size_t)min(s, (int)gridDim.y - 1) * M * rank + at);
+      float v = p[0];
+#pragma unroll
+      for (int s = 1; s < kXaSlabs; ++s) v += s < (int)gridDim.y ? p[s] : 0.0f;
+      xa[at] = v;
+    }
+    if (tid == 0) __hip_atomic_store(&counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// bf16 rows past the skinny kernel's, with room for the slabs' partials.  One
+// workgroup reads its whole factor, 4 K rank bytes, through its CU's 64 bytes
+// a cycle (8192 x 64: 14 us), whatever the rows; from 2^18 factor elements
+// four slabs of K, and as many rows a group as keep the grid within a
+// workgroup a CU, cost less than their hand-off.  Adapted linears as a whole,
+// one slab -> four, at 65 / 128 / 192 rows: 4096 -> 4096 rank 64 30 / 36 / 38
+// -> 26 / 31 / 35 us, 8192 -> 2048 rank 32 30 / 35 / 35 -> 26 / 31 / 33, rank
+// 64 40 / 43 / 44 -> 28 / 32 / 37; but rank 16 26 / 30 / 30 -> 25 / 29 / 32.
+template <int VEC>
+void launch_xa_slabs(const uint16_t* x, const float* a, int M, int K, int rank, float* xa, float* part,
+                     unsigned* counters, hipStream_t stream) {
+  int lpk = 1;
+  while (lpk * VEC < rank) lpk <<= 1;
+  const int kslab = (K + kXaSlabs - 1) / kXaSlabs;
+  const unsigned slabs = (unsigned)((K + kslab - 1) / kslab);  // no empty slab
+  if (M <= 128)
+    lora_xa_kernel<true, VEC, 2, true><<<dim3((unsigned)(M + 1) / 2, slabs), kXaThreads, 0, stream>>>(
+        x, a, M, K, rank, lpk, (size_t)rank, 1, xa, kslab, part, counters);
+  else
+    lora_xa_kernel<true, VEC, 4, true><<<dim3((unsigned)(M + 3) / 4, slabs), kXaThreads, 0, stream>>>(
+        x, a, M, K, rank, lpk, (size_t)rank, 1, xa, kslab, part, counters);
 }
 
 template <bool XBF16, int VEC>
@@ -190,7 +243,8 @@ void launch_xa(const void* x, const float* a, int M, int K, int rank, size_t sk,
   // 48; 4096 -> 4096 at 100 rows 25.7 against 30).  Past that, four rows share
   // each factor load.
   if (M <= 256) {
-    lora_xa_kernel<XBF16, VEC, 1><<<M, kXaThreads, 0, stream>>>(x, a, M, K, rank, lpk, sk, sj, xa);
+    lora_xa_kernel<XBF16, VEC, 1, false><<<M, kXaThreads, 0, stream>>>(x, a, M, K, rank, lpk, sk, sj, xa, 0, nullptr,
+                                                                       nullptr);
     return;
   }
   // at most kXaRows rows a launch: the work items of one past 2^32 wrap
@@ -200,8 +254,8 @@ void launch_xa(const void* x, const float* a, int M, int K, int rank, size_t sk,
   for (int64_t m = 0; m < M; m += kXaRows) {
     const int rows = (int)std::min<int64_t>(kXaRows, M - m);
     const void* xm = static_cast<const char*>(x) + (size_t)m * K * (XBF16 ? 2 : 4);
-    lora_xa_kernel<XBF16, VEC, 4><<<(rows + 3) / 4, kXaThreads, 0, stream>>>(xm, a, rows, K, rank, lpk, sk, sj,
-                                                                          xa + (size_t)m * rank);
+    lora_xa_kernel<XBF16, VEC, 4, false><<<(rows + 3) / 4, kXaThreads, 0, stream>>>(
+        xm, a, rows, K, rank, lpk, sk, sj, xa + (size_t)m * rank, 0, nullptr, nullptr);
   }
 }
 
@@ -473,6 +527,21 @@ hipError_t launch_lora_xa_strided(const void* x, bool x_bf16, const float* a, si
     if (vec) launch_xa<false, 4>(x, a, M, K, rank, sk, sj, xa, stream);
     else launch_xa<false, 1>(x, a, M, K, rank, sk, sj, xa, stream);
   }
+  return hipGetLastError();
+}
+
+size_t lora_xa_slab_floats(int M, int K, int rank) {
+  return M <= 256 && (int64_t)K * rank >= 1 << 18 ? (size_t)kXaSlabs * M * rank : 0;
+}
+
+hipError_t launch_lora_xa_slabs(const uint16_t* x, const float* a, int M, int K, int rank, float* xa, float* part,
+                                unsigned* counters, hipStream_t stream) {
+  if (rank < 1 || rank > 64 || M < 1 || lora_xa_slab_floats(M, K, rank) == 0) return hipErrorInvalidValue;
+  // four columns a lane where every factor row is four-float aligned
+  if (rank % 4 == 0 && (reinterpret_cast<uintptr_t>(a) & 15u) == 0)
+    launch_xa_slabs<4>(x, a, M, K, rank, xa, part, counters, stream);
+  else
+    launch_xa_slabs<1>(x, a, M, K, rank, xa, part, counters, stream);
   return hipGetLastError();
 }
 

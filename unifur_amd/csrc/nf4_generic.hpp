@@ -20,6 +20,12 @@ hipError_t launch_gemm_f32(const void* x, bool x_bf16, const float* w, int M, in
                            hipStream_t stream);
 hipError_t launch_lora_xa(const void* x, bool x_bf16, const float* a, int M, int K, int rank, float* xa,
                           hipStream_t stream);
+// x A of 5 to 256 bf16 rows, a [K][rank], in slabs of K over more workgroups:
+// part holds lora_xa_slab_floats(M, K, rank) floats (0: not for this shape),
+// counters a zeroed unsigned per row, left zero.
+size_t lora_xa_slab_floats(int M, int K, int rank);
+hipError_t launch_lora_xa_slabs(const uint16_t* x, const float* a, int M, int K, int rank, float* xa, float* part,
+                                unsigned* counters, hipStream_t stream);
 // y = x w^T with w stored [N, K] (same epilogue).
 hipError_t launch_gemm_f32_wt(const void* x, bool x_bf16, const float* wt, int M, int K, int N, const Epilogue& e,
                               hipStream_t stream);
