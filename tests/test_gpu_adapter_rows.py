@@ -1,9 +1,9 @@
 """The adapter term of decode-sized calls, (x A) B s (LoraAdapter::forward,
 src/quantize.rs:619-624), alone over an all-zero base weight: the x A kernel
-at one and four rows per workgroup, a last row group that is not full, every
-lane split of the rank (powers of two, ranks between them, factors that are
-not four-float aligned), d_in below and past one step of the workgroup, and
-the epilogue's batches of sixteen ranks with a remainder.
+at one row per workgroup and, past 256 rows, at four with a last row group that
+is not full, every lane split of the rank (powers of two, ranks between them,
+factors that are not four-float aligned), d_in below and past one step of the
+workgroup, and the epilogue's batches of sixteen ranks with a remainder.
 
 x is exact in its dtype and everything after it is f32, so both activation
 types are held to the f32 bar (1e-5 of the sum of |products|).
@@ -51,6 +51,25 @@ def test_adapter_term_with_a_factor_off_sixteen_bytes(device, oracle, shift):
     got = Q.QloraLinear(lin, ad).forward(xt).cpu().numpy().astype(np.float64)
     bound = (np.abs(x) @ np.abs(a)) @ np.abs(b) * s
     assert float(np.max(np.abs(got - oracle.lora_ref_f64(x, a, b, s)) / bound)) <= TOL_F32
+
+
+# past 256 rows, where no other kernel takes x A: a dense f32 linear (f32 and
+# bf16 x), and a d_in the row products refuse (no multiple of 8) through the f32 GEMM
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [257, 259, 260])
+@pytest.mark.parametrize("K,r", [(12, 4), (300, 16), (1032, 7)])
+def test_four_rows_a_workgroup(device, oracle, dt, rows, K, r):
+    N, s = 192, 0.5
+    x, xt = acts(oracle, rows, K, 0x96 + K, dt, device)
+    a, b, ad = lora_parts(oracle, K, N, r, 0x97 + r, device, scaling=s, sigma=0.05)
+    ref = oracle.lora_ref_f64(x, a, b, s)
+    bound = (np.abs(x) @ np.abs(a)) @ np.abs(b) * s
+    layers = [Q.QLoRALinear(Q.DenseLinear(torch.zeros(K, N, device=device)), ad, K * N, False)]
+    if dt == torch.float32 and K % 8:
+        layers.append(Q.QloraLinear(zero_linear(K, N, device, True), ad))
+    for layer in layers:
+        got = layer.forward(xt, out_dtype=torch.float32).cpu().numpy().astype(np.float64)
+        assert float(np.max(np.abs(got - ref) / bound)) <= TOL_F32
 
 
 def test_rows_past_one_launch(device):

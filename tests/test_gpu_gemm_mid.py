@@ -100,3 +100,52 @@ def test_an_adapter_of_zeros_adds_nothing(device, oracle):
     _, xt = acts(oracle, 100, K, 0xC5, torch.bfloat16, device)
     fresh = Q.LoraAdapter.new(Q.LoraConfig.new(K, N, 16), device=device)
     assert torch.equal(Q.QloraLinear(lin, fresh).forward(xt), lin.forward(xt))
+
+
+# 2^25 weights and more: up to 256 rows
+@pytest.mark.parametrize("rows,K,N", [(193, 4096, 8192), (256, 4096, 8192), (224, 11008, 4096)])
+def test_rows_past_192(device, oracle, rows, K, N):
+    lin, wdeq = make_linear(oracle, K, N, 0xC9, device)
+    x, xt = acts(oracle, rows, K, 0xCA, torch.bfloat16, device)
+    ref = oracle.linear_ref_f64(x, wdeq)
+    lib = L.lib()
+    full = lib.unifur_nf4_linear_workspace_size(rows, K, N, L.BF16, 0)
+    y = forward(lin, xt, rows, None, None, torch.empty(rows, N, device=device), full)
+    check(y, ref, x, wdeq, TOL_BF16, f"mid {rows} x {K} -> {N}")
+    least = lib.unifur_nf4_linear_min_workspace_size(rows, K, N, L.BF16, 0)
+    assert torch.equal(y, forward(lin, xt, rows, None, None, torch.empty(rows, N, device=device), least))
+
+
+# the SwiGLU block's down projection takes this kernel over a striped weight of
+# 2^24 values or more; its slabs lie in the block's partials
+@pytest.mark.parametrize("hidden,inter", [(4096, 11008), (2048, 8192)])
+@pytest.mark.parametrize("dq", [True, False])
+@pytest.mark.parametrize("rows", [65, 129, 192, 256])
+def test_swiglu_down(device, hidden, inter, dq, rows):
+    g = torch.Generator(device)
+    g.manual_seed(0xCB)
+    lins = []
+    for k, n in ((hidden, inter), (hidden, inter), (inter, hidden)):
+        p = Q.PackedNf4Tensor.quantize(torch.randn(k * n, generator=g, device=device) * 0.02)
+        lins.append(Q.Nf4Linear.from_packed(p.with_double_quantization() if dq else p, k, n, striped=True))
+    x = torch.randn(rows, hidden, generator=g, device=device).bfloat16()
+    wg, wu, wd = [m.dequantized_weight().double().view(m.d_input(), m.d_output()) for m in lins]
+    a = x.double() @ wg
+    h = a * torch.sigmoid(a) * (x.double() @ wu)
+    ref, bound = h @ wd, h.abs() @ wd.abs()
+    ws3 = [m.weight_struct() for m in lins]
+    lib = L.lib()
+    full = lib.unifur_nf4_swiglu_workspace_size(rows, hidden, inter, L.BF16)
+    least = lib.unifur_nf4_swiglu_min_workspace_size(rows, hidden, inter, L.BF16)
+    buf = torch.full((rows * hidden + 8,), float("nan"), device=device)
+    for need, shift in ((full, 0), (least, 0), (full, 1)):  # shift: an output off 16 bytes
+        y = buf[shift:shift + rows * hidden].view(rows, hidden)
+        ws = torch.zeros(need, dtype=torch.uint8, device=device)
+        L.check(lib.unifur_nf4_swiglu_forward(x.data_ptr(), L.BF16, rows, *[ctypes.byref(w) for w in ws3],
+                                              y.data_ptr(), L.F32, ws.data_ptr(), need,
+                                              torch.cuda.current_stream().cuda_stream))
+        e = (y.double() - ref).abs()
+        assert float((e / bound).max()) <= TOL_BF16 and float(e.max() / ref.abs().max()) <= TOL_BF16
+        assert int(ws[:65536].count_nonzero()) == 0
+        assert torch.isnan(buf[shift + rows * hidden:]).all()
+        buf.fill_(float("nan"))
