@@ -36,7 +36,6 @@ if ROOT not in sys.path:
 METRIC = "NF4 dequant/GEMV GB/s and prefill GEMM TFLOP/s, % of MI355X roofline"
 HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2516.6
-F32_MFMA_PEAK_TFLOPS = 157.3
 MALL_BYTES = 256 << 20
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_gemv_config2.txt")
 
@@ -593,9 +592,12 @@ def bench_gemm(torch, Q, L) -> dict:
     dx_launch(0)
     gdx = capture(torch, dx_launch, 4)
     msdx = steady_ms(torch, gdx, 4, reps=5) if gdx is not None else event_ms(torch, dx_launch, 8)
-    f32 = {"path": "f32 MFMA (v_mfma_f32_32x32x2f32) over NF4 tiles dequantized exactly in LDS",
+    # the f32 GEMM forms each base product from six bf16 products, so its time
+    # is priced against the bf16 matrix-core peak
+    f32 = {"path": "f32 GEMM, six bf16 products (v_mfma_f32_32x32x16_bf16) per f32 product, NF4 dequantized "
+                   "exactly in registers",
            "qlora_ms": round(ms32, 5), "qlora_tflops": round(flops / ms32 / 1e9, 1),
-           "frac_of_f32_mfma_peak": round(flops / ms32 / 1e9 / F32_MFMA_PEAK_TFLOPS, 4),
+           "bf16_products_frac_of_peak": round(6 * base_flops / ms32 / 1e9 / BF16_PEAK_TFLOPS, 4),
            "backward_dx_ms": round(msdx, 5), "backward_dx_tflops": round(base_flops / msdx / 1e9, 1),
            "max_rel_err": e32}
     return {"ms": ms, "tflops": flops / ms / 1e9, "frac": flops / ms / 1e9 / BF16_PEAK_TFLOPS,

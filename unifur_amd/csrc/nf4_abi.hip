@@ -246,12 +246,16 @@ struct LinearLayout {
 
 // Decode-sized batches (<= 4 rows) take a GEMV (the striped one for striped
 // weights); bf16 batches up to 64 rows over a striped weight the skinny MFMA
-// kernel; larger bf16 batches the prefill path: with `expand`, the weight
-// (plus the LoRA update) expanded once to bf16 in the workspace and a BLAS
-// GEMM, else the fused MFMA kernel that dequantizes W tiles in LDS (no
-// weight-sized scratch); everything else the generic dequantize + f32
-// matmul (a striped weight is first put back in row-major order in the
-// workspace).
+// kernel; bf16 batches past that over a large striped weight, up to 192 or 256
+// rows, the mid kernel (with `mid`), which dequantizes W in the registers that
+// feed its MFMAs; larger bf16 batches the prefill path: with `expand`, the
+// weight (plus the LoRA update) expanded once to bf16 in the workspace and a
+// BLAS GEMM, else the fused MFMA kernel that dequantizes W tiles in LDS (no
+// weight-sized scratch).  f32 batches take the skinny kernel up to 32 rows (64
+// where d_in is short) and past it the f32 GEMM over the exact weight, as do
+// bf16 batches whose d_in the bf16 kernels do not take; everything else the
+// generic dequantize + f32 matmul (a striped weight is first put back in
+// row-major order in the workspace).
 LinearLayout plan_linear(uint64_t rows, uint64_t d_in, uint64_t d_out, uint32_t lora_rank, const void* packed,
                          int x_dtype, const void* x, bool striped, int scale_kind, bool expand = true,
                          bool split = true, bool mid = true) {
@@ -329,8 +333,8 @@ LinearLayout plan_linear(uint64_t rows, uint64_t d_in, uint64_t d_out, uint32_t 
   } else if (f32_gemm ||
              (xf32 && rows <= 0x7fffffffu && d_in <= 0x7fffffffu && d_out <= 0x7fffffffu && aligned_to(packed, 8) &&
               gemm_f32_mfma_supported((int)rows, (int)d_in, (int)d_out, (int)d_out, x))) {
-    // f32 activations past the skinny kernel: the f32 MFMA kernel over W
-    // tiles dequantized in LDS (no weight-sized scratch)
+    // f32 activations past the skinny kernel: the f32 GEMM, W dequantized
+    // exactly in the registers that feed its MFMAs (no weight-sized scratch)
     L.path = LinearPath::kMfmaF32;
     if (split) {  // partials of its K slabs (without them a workgroup takes the slabs in turn)
       L.splits = gemm_f32_splits((int)rows, (int)d_in, (int)d_out);
@@ -1278,7 +1282,7 @@ int run_backward(const void* dy, int dy_dtype, uint64_t rows, const unifur_nf4_w
       a.lora_scaling = lora ? lora->scaling : 0.0f;
       a.y = dx;
       a.y_bf16 = dx_dtype == UNIFUR_NF4_BF16;
-        a.partials = L.splits > 1 ? at<float>(ws, L.dx_partials) : nullptr;
+      a.partials = L.splits > 1 ? at<float>(ws, L.dx_partials) : nullptr;
       UNIFUR_HIP(launch_gemm_f32_mfma(a, w->scales.kind == UNIFUR_NF4_SCALES_DOUBLE_QUANTIZED, is_striped(w), true,
                                       stream));
     } else {

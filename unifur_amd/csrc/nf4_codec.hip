@@ -456,8 +456,8 @@ int grid_for(size_t work_items, int threads, int max_blocks) {
 //      holding K rows of 8 bytes, so a span writes 128 contiguous bytes per
 //      stripe -- and its f32 absmax to absmax_tmp[b K + k], the striped
 //      scale order
-//   2. the max of each tensor's block scales (one workgroup per tensor; an
-//      atomic max per wave instead serialises on one address per tensor)
+//   2. the max of each tensor's block scales (up to sixteen workgroups a
+//      tensor with one atomic max each, on bits that step 1 cleared)
 //   3. encode absmax_tmp against the max into the u8 scales, same order
 constexpr int kQGroupMax = 48;
 
