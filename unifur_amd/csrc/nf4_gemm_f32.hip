@@ -39,12 +39,14 @@
 // there are three of them: the path of bf16 batches whose shape the bf16
 // kernels do not take, where the weight stays the exact f32 one.
 //
-// What bounds it: at 2048 x 4096 -> 4096, 370 us (601 with the f32
-// instruction), the matrix cores' power: 1.1 PFLOP/s of bf16 products, what a
-// large bf16 product reaches here.  500 rows take 110 us (366 with the f32
-// instruction, whose 128 tiles left half the CUs idle; now four slabs of K):
-// 0.9 PFLOP/s, the rest being the slabs' partials, 33 MB written and read, the
-// reduction launch, and the weight decoded and cut once per 128 rows.  The
+// What bounds it (counters in profiles/mfma_utilisation_prefill.txt): 2048 x
+// 4096 -> 4096 in 370 us (601 with the f32 instruction) is 1.1 PFLOP/s of bf16
+// products, what the library's large bf16 product reaches here, with the matrix
+// cores busy 51 % of the cycles of a clock that falls to 2.1 GHz (its own: 50 %).
+// 500 rows take 110 us (366 with the f32 instruction, whose 128 tiles left half
+// the CUs idle; now four slabs of K): 0.9 PFLOP/s, busy 42 %; the slabs'
+// partials, 33 MB written and read, take a 7 us reduction launch and part of the
+// kernel's time, and the weight is decoded and cut once per 128 rows.  The
 // second accumulator costs registers (134 -> 205 at 128 rows, two workgroups a
 // CU) but no time: 2048 rows 380 us with one and 370 with two, 500 rows 112
 // and 110, 1024 x 4096 -> 11008 606 and 577, 64 x 4096 -> 11008 52 and 51.

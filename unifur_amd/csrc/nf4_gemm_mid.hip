@@ -25,9 +25,10 @@
 // (gemm_mid_wanted has the rest).
 //
 // What bounds it: one wave a SIMD issues its VALU, LDS and MFMA work one after
-// the other (counters at 128 x 4096 -> 32768: matrix cores busy 23 % of the
-// cycles, VALU 21 %, LDS instructions 14 %, waiting 30 %), 1850 cycles a step
-// where the MFMAs need 512; deeper prefetch and LDS reads spread between the
+// the other (counters at 128 x 4096 -> 32768, 54 us, in
+// profiles/mfma_utilisation_prefill.txt: matrix cores busy 25 % of the cycles,
+// VALU 28 %, LDS 16 %, waiting 25 %), 2050 cycles a step where the MFMAs need
+// 512; deeper prefetch and LDS reads spread between the
 // MFMAs measured the same, two workgroups a CU cost in partials what they
 // gain.
 #include "nf4_gemm_mid.hpp"
