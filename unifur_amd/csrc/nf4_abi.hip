@@ -638,7 +638,7 @@ struct MlpLayout {
   int split_up = 1, split_down = 1;  // kMfma without expand: d_in slabs of the fused kernel
   int tail_up = 1, tail_down = 1;    // ... or of only its last, partly filled round of tiles
   int mid_down = 0;                  // kMfma without expand: d_in slabs of down on the mid-size kernel (0: not taken)
-  bool f32_mfma = false;             // kGeneric with f32 activations: the f32 MFMA kernel per linear
+  bool f32_mfma = false;             // kGeneric: the f32 GEMM per linear
   size_t partials0, partials1, h, u, hb, wt, blas, wf32, rm_codes, rm_scales, gemm_partials, total;
 };
 
@@ -1064,7 +1064,7 @@ Branch branch_for(hipStream_t stream) {
 struct BackwardLayout {
   bool blas, fused;
   int splits;  // fused dX: d_out slabs (1: none)
-  bool mfma_f32;  // f32 dY: the f32 MFMA kernel over W's rows (dY B^T in dy_bt when there is an adapter)
+  bool mfma_f32;  // f32 dY: the f32 GEMM over W's rows (dY B^T in dy_bt when there is an adapter)
   size_t dy_bt;
   size_t wt, blas_ws, wf32, rm_codes, rm_scales, lora_at, lora_bt, lora_xa, dx_partials, grads, xa, u, partials, total;
 };
@@ -1104,7 +1104,7 @@ BackwardLayout plan_backward(uint64_t rows, uint64_t d_in, uint64_t d_out, uint3
     } else if (dy_dtype == UNIFUR_NF4_F32 && aligned && codes_aligned && sizes && d_out % 64 == 0 &&
                gemm_f32_mfma_supported((int)rows, (int)d_out, (int)d_in, (int)d_out,
                                        reinterpret_cast<const void*>(uintptr_t{256}))) {
-      // f32 dY: dX on the f32 MFMA kernel with W's rows as its outputs
+      // f32 dY: dX on the f32 GEMM with W's rows as its outputs
       L.mfma_f32 = true;
       if (allow_split) {
         L.splits = gemm_f32_splits((int)rows, (int)d_out, (int)d_in);
