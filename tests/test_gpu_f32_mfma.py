@@ -2,9 +2,9 @@
 QloraLinear::forward (src/qwennet.rs:238-241, :325-345) with f32 activations
 past the skinny kernel's rows, the backward's dX for f32 dY (the autodiff
 under src/qwentrain.rs:421-470), and the SwiGLU block (src/qwennet.rs:816-819)
-with f32 activations -- the reference's own f32 arithmetic, now on
-v_mfma_f32_32x32x2f32 with the weight dequantized exactly in LDS instead of
-an f32 copy of the whole weight.
+with f32 activations -- the reference's own f32 arithmetic, each product from
+six bf16 ones, with the weight dequantized exactly in registers instead of an
+f32 copy of the whole weight.
 
 Each case is checked against the float64 product of the same inputs with the
 oracle's dequantized weight at the f32 bar (1e-5, normwise over the summed

@@ -125,3 +125,40 @@ def test_least_workspace_and_capture_take_the_slabs_in_turn(device, oracle):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, y)
+
+
+def call(lin, xt, need, adapter=None):
+    y = torch.empty(xt.shape[0], lin.d_output(), device=xt.device)
+    ws = torch.zeros(need, dtype=torch.uint8, device=xt.device)
+    w, lo = lin.weight_struct(), adapter.struct() if adapter is not None else None
+    L.check(L.lib().unifur_nf4_linear_forward(xt.data_ptr(), L.F32, xt.shape[0], ctypes.byref(w), None,
+                                              ctypes.byref(lo) if lo is not None else None, y.data_ptr(), L.F32,
+                                              ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+    return y
+
+
+def in_skinny_launches(lin, xt, adapter=None):
+    """What launches of at most 32 rows give, each by a call of its own."""
+    layer = Q.QloraLinear(lin, adapter) if adapter is not None else lin
+    return torch.cat([layer.forward(xt[m:m + 32]) for m in range(0, xt.shape[0], 32)])
+
+
+@pytest.mark.parametrize("rows", [40, 64])
+@pytest.mark.parametrize("K,N,r", [(4096, 4096, 0), (2048, 8192, 8), (11008, 256, 0)])
+def test_without_room_33_to_64_rows_take_the_skinny_kernel(device, oracle, rows, K, N, r):
+    """One workgroup a tile taking the slabs in turn is several times slower
+    there than two skinny launches."""
+    lin, wdeq = make_linear(oracle, K, N, 0xBB, device)
+    x, xt = acts(oracle, rows, K, 0xBC, torch.float32, device)
+    w = wdeq.astype(np.float64)
+    ref, bound, ad = x.astype(np.float64) @ w, np.abs(x) @ np.abs(w), None
+    if r:
+        a, b, ad = lora_parts(oracle, K, N, r, 0xBD, device)
+        ref = ref + oracle.lora_ref_f64(x, a, b, 2.0)
+        bound = bound + (np.abs(x) @ np.abs(a)) @ np.abs(b) * 2.0
+    lib = L.lib()
+    y = call(lin, xt, lib.unifur_nf4_linear_min_workspace_size(rows, K, N, L.F32, r), ad)
+    assert torch.equal(y, in_skinny_launches(lin, xt, ad))
+    assert worst(y.cpu().numpy(), ref, bound) <= TOL_F32
+    full = call(lin, xt, lib.unifur_nf4_linear_workspace_size(rows, K, N, L.F32, r), ad)
+    assert worst(full.cpu().numpy(), ref, bound) <= TOL_F32

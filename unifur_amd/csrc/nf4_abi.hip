@@ -176,9 +176,10 @@ int resolve_workspace(void* user, uint64_t user_bytes, size_t need, hipStream_t 
 // Whether a call's workspace can hold `need` bytes: the caller's as it is,
 // the internal one after growing to them (not under capture, nor when the
 // device is out of memory).  For the f32 GEMM's slab partials, without which
-// its call gives the same bits: the only plan whose internal workspace may
-// turn out smaller (every other one is refused under capture, so that a graph
-// never holds a slower form unnoticed).  Leaves no error text behind.
+// its call goes on (to the same bits past 64 rows; 33 to 64 take the skinny
+// kernel): the only plan whose internal workspace may turn out smaller (every
+// other one is refused under capture, so that a graph never holds a slower
+// form unnoticed).  Leaves no error text behind.
 bool workspace_holds(void* user, uint64_t user_bytes, size_t need, hipStream_t stream) {
   if (user) return user_bytes >= need;
   const std::string text = g_last_error;
@@ -275,12 +276,14 @@ LinearLayout plan_linear(uint64_t rows, uint64_t d_in, uint64_t d_out, uint32_t 
   const bool xf32 = x_dtype == UNIFUR_NF4_F32;
   const uint64_t sk_rows = xf32 ? std::min<uint64_t>(rows, kSkinnyMaxRowsF32) : rows;
   // past one skinny launch the f32 GEMM's 64-row tile, where d_in gives it
-  // slabs to fill the chip (4096 -> 11008 at 33 / 64 rows 51 / 54 us against
-  // 70 / 91 of two skinny launches, 4864 -> 896 22 / 24 against 27; but
-  // 896 -> 4864 19 / 22 against 17 / 22)
+  // slabs to fill the chip and there is room for their partials (33 / 64 rows
+  // against two skinny launches: 4096 -> 11008 48 / 52 us against 68 / 89,
+  // 4864 -> 896 22 / 24 against 26 / 26; 896 -> 4864 19 / 22 against 17 / 22;
+  // in turn 4096 -> 4096 146 / 149 against 31 / 40)
   const bool f32_gemm = xf32 && rows > (uint64_t)kSkinnyMaxRowsF32 && d_in >= 2048 && rows <= 0x7fffffffu &&
                         d_in <= 0x7fffffffu && d_out <= 0x7fffffffu && aligned_to(packed, 8) &&
-                        gemm_f32_mfma_supported((int)rows, (int)d_in, (int)d_out, (int)d_out, x);
+                        gemm_f32_mfma_supported((int)rows, (int)d_in, (int)d_out, (int)d_out, x) &&
+                        (split || gemm_f32_splits((int)rows, (int)d_in, (int)d_out) == 1);
   const bool skinny = !small && striped && !f32_gemm && rows <= (uint64_t)kSkinnyMaxRows && d_in <= 0x7fffffffu &&
                       skinny_supported((int)sk_rows, (int)d_in, x, xf32) && d_out / 64 <= (uint64_t)kMaxCounters;
   if (small && striped) {
