@@ -16,6 +16,7 @@ import torch
 from unifur_amd import _lib as L
 from unifur_amd import quantize as Q
 
+from test_gpu_capture_workspace import captured, stream  # noqa: F401 (a fixture)
 from test_gpu_gemm import lora_parts, zero_linear
 from test_gpu_linear import TOL_BF16, TOL_F32, acts, check, make_linear
 
@@ -149,3 +150,22 @@ def test_swiglu_down(device, hidden, inter, dq, rows):
         assert int(ws[:65536].count_nonzero()) == 0
         assert torch.isnan(buf[shift + rows * hidden:]).all()
         buf.fill_(float("nan"))
+
+
+@pytest.mark.parametrize("K,N", [(4096, 4096), (8192, 2048)])
+def test_a_workspace_between_takes_the_fused_slabs(device, oracle, stream, K, N):
+    """128 rows in 16 MiB: the fused kernel's slabs fit where this kernel's
+    just do not; a split launch and its reduction, not one launch of workgroups
+    that take the slabs in turn (two to three times slower)."""
+    h, s = stream
+    rows, need = 128, 16 << 20
+    lin, wdeq = make_linear(oracle, K, N, 0xCC, device)
+    x, xt = acts(oracle, rows, K, 0xCD, torch.bfloat16, device)
+    y = forward(lin, xt, rows, None, None, torch.empty(rows, N, device=device), need)
+    check(y, oracle.linear_ref_f64(x, wdeq), x, wdeq, TOL_BF16, f"{rows} x {K} -> {N} in 16 MiB")
+    ws, w = torch.zeros(need, dtype=torch.uint8, device=device), lin.weight_struct()
+    torch.cuda.synchronize()
+    for room, launches in ((need, 2), (L.lib().unifur_nf4_linear_min_workspace_size(rows, K, N, L.BF16, 0), 1)):
+        st, text, nodes = captured(h, s, lambda: L.lib().unifur_nf4_linear_forward(
+            xt.data_ptr(), L.BF16, rows, ctypes.byref(w), None, None, y.data_ptr(), L.F32, ws.data_ptr(), room, s))
+        assert (st, nodes) == (L.OK, launches), (st, nodes, text)

@@ -467,7 +467,18 @@ int run_linear(const void* x, int x_dtype, uint64_t rows, const unifur_nf4_weigh
       L.gemm_partials = 0;
       L.total = L.lean;
     }
-    if (workspace) {
+    if (workspace && L.splits > 1 && !L.gemm_partials) {
+      // room for the fused kernel's split-K partials, if not for these: its
+      // slabs beat a workgroup a tile taking them in turn (128 rows in the
+      // static 16 MiB: 4096 -> 4096 28 against 55 us, 8192 -> 2048 29 against
+      // 104, 2048 -> 8192 24 against 30)
+      const LinearLayout fused = plan_linear(rows, w->d_in, w->d_out, rank, w->packed, x_dtype, x, true,
+                                             w->scales.kind, false, true, false);
+      if (fused.path == LinearPath::kMfma && fused.gemm_partials && aligned_to(y, 16) && aligned_to(bias, 16) &&
+          workspace_bytes >= fused.total)
+        L = fused;
+    }
+    if (workspace && L.path == LinearPath::kMid) {
       // no room for x A, or less than the other paths accept: their plan
       // (which refuses the latter)
       const LinearLayout other = plan_linear(rows, w->d_in, w->d_out, rank, w->packed, x_dtype, x, true,
