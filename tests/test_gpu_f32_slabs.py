@@ -162,3 +162,14 @@ def test_without_room_33_to_64_rows_take_the_skinny_kernel(device, oracle, rows,
     assert worst(y.cpu().numpy(), ref, bound) <= TOL_F32
     full = call(lin, xt, lib.unifur_nf4_linear_workspace_size(rows, K, N, L.F32, r), ad)
     assert worst(full.cpu().numpy(), ref, bound) <= TOL_F32
+
+
+@pytest.mark.parametrize("rows", [40, 64])
+@pytest.mark.parametrize("K,N", [(8192, 256), (16384, 896), (2048, 8192)])
+def test_narrow_and_one_round_shapes_stay_on_the_skinny_kernel(device, oracle, rows, K, N):
+    lin, wdeq = make_linear(oracle, K, N, 0xBE, device)
+    x, xt = acts(oracle, rows, K, 0xBF, torch.float32, device)
+    w = wdeq.astype(np.float64)
+    y = lin.forward(xt)
+    assert torch.equal(y, in_skinny_launches(lin, xt))
+    assert worst(y.cpu().numpy(), x.astype(np.float64) @ w, np.abs(x) @ np.abs(w)) <= TOL_F32

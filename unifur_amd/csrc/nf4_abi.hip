@@ -276,11 +276,22 @@ LinearLayout plan_linear(uint64_t rows, uint64_t d_in, uint64_t d_out, uint32_t 
   const bool xf32 = x_dtype == UNIFUR_NF4_F32;
   const uint64_t sk_rows = xf32 ? std::min<uint64_t>(rows, kSkinnyMaxRowsF32) : rows;
   // past one skinny launch the f32 GEMM's 64-row tile, where d_in gives it
-  // slabs to fill the chip and there is room for their partials (33 / 64 rows
-  // against two skinny launches: 4096 -> 11008 48 / 52 us against 68 / 89,
-  // 4864 -> 896 22 / 24 against 26 / 26; 896 -> 4864 19 / 22 against 17 / 22;
-  // in turn 4096 -> 4096 146 / 149 against 31 / 40)
-  const bool f32_gemm = xf32 && rows > (uint64_t)kSkinnyMaxRowsF32 && d_in >= 2048 && rows <= 0x7fffffffu &&
+  // slabs to fill the chip and there is room for their partials.  33 / 64 rows
+  // against two skinny launches: 2048 -> 2048 18 / 20 us against 18 / 23,
+  // 4096 -> 11008 48 / 52 against 68 / 89, 4864 -> 896 22 / 24 against 26 / 26,
+  // 11008 -> 4096 47 / 51 against 60 / 76.  Not where
+  //   d_in is short: 896 -> 4864 19 / 22 against 17 / 22;
+  //   few columns leave only its sixteen slabs, where the skinny kernel splits
+  //   a long d_in further: 6144 -> 256 23 / 25 against 26 / 26, but 8192 -> 256
+  //   27 / 30 against 22 / 23, 16384 -> 512 44 / 46 against 27 / 31;
+  //   the skinny grid is one full round over a d_in that needs no slabs:
+  //   2048 -> 4096 19 / 23 against 18 / 23, 2048 -> 8192 27 / 33 against
+  //   25 / 32 (2048 -> 11008 31 / 35 against 40 / 52);
+  //   the slabs go in turn: 4096 -> 4096 146 / 149 against 31 / 40.
+  const bool narrow = striped && d_out < 1024 && d_in > 6144;
+  const bool one_round = striped && d_in < 2560 && d_out >= 4096 && d_out <= 8192;
+  const bool f32_gemm = xf32 && rows > (uint64_t)kSkinnyMaxRowsF32 && d_in >= 2048 && !narrow && !one_round &&
+                        rows <= 0x7fffffffu &&
                         d_in <= 0x7fffffffu && d_out <= 0x7fffffffu && aligned_to(packed, 8) &&
                         gemm_f32_mfma_supported((int)rows, (int)d_in, (int)d_out, (int)d_out, x) &&
                         (split || gemm_f32_splits((int)rows, (int)d_in, (int)d_out) == 1);
