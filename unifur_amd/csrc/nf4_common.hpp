@@ -33,6 +33,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int v2i32 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
@@ -100,6 +102,23 @@ __device__ __forceinline__ uint32_t dpp_mov(uint32_t v) {
                 "a DPP pattern with out-of-range source lanes");
   return __builtin_amdgcn_update_dpp(0u, v, CTRL, 0xF, 0xF, true);
 }
+
+// The value of lane 16 (l / 16) + J, and of all sixteen.
+template <int J>
+__device__ __forceinline__ float row_lane(float v) {
+  return __uint_as_float(dpp_mov<0x150 + J>(__float_as_uint(v)));
+}
+template <int J>
+__device__ __forceinline__ void row_lanes(float v, float (&o)[16]) {
+  o[J] = row_lane<J>(v);
+  if constexpr (J + 1 < 16) row_lanes<J + 1>(v, o);
+}
+
+// LDS addressed by byte offset.
+typedef __attribute__((address_space(3))) v2i32 lds_v2i32;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) const f32x2 lds_f32x2_c;
 
 // Split-K hand-off between workgroups.  Partial sums are written with
 // agent-scope atomic stores (coherent across the XCDs' L2s) and the writer

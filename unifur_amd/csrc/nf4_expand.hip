@@ -33,7 +33,6 @@ constexpr int kLdsBytes = 256;                        // LDS bytes: the four wav
 constexpr int kMaxRank = 64;
 constexpr int kRowPitch = 144;                    // LDS bytes per row of a ROWS tile (64 bf16 + 16: two-way banks)
 constexpr int kRowTileBytes = 64 * kRowPitch;
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 struct ExpandArgs {
   const uint8_t* packed;
@@ -360,7 +359,6 @@ hipError_t launch_layout(const ExpandArgs& a, bool dq, bool striped, int n_count
 bool expand_supported(int K, int N, int rank) {
   return K > 0 && N > 0 && K % kTile == 0 && N % kTile == 0 && rank >= 0 && rank <= kMaxRank;
 }
-
 
 hipError_t launch_expand_bf16(const uint8_t* packed, const ScalesArg& scales, int K, int N, bool striped,
                               const float* lora_a, const float* lora_b, int rank, float scaling, uint16_t* wt,

@@ -54,11 +54,7 @@ constexpr int kLdsDq = kLdsLut + kLutBytes;      // DQ scale LUTs, 256 x f32 per
 constexpr size_t kGemmSmem = kLdsDq + 2 * 256 * 4;  // 148 KiB: one workgroup per CU
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
-typedef __attribute__((address_space(3))) const f32x2 lds_f32x2_c;
 
 struct GemmArgs {
   const uint16_t* x;  // [M, K] bf16

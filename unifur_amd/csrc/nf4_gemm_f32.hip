@@ -73,13 +73,6 @@ namespace {
 constexpr int kFN = 128, kFK = 32;
 constexpr int kFThreads = 256;
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef int v2i32 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) v2i32 lds_v2i32;
-typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-typedef __attribute__((address_space(3))) const f32x2 lds_f32x2_c;
-
 // LDS of a workgroup of RT row tiles (byte offsets).
 template <int RT>
 struct FSmem {
@@ -130,16 +123,6 @@ __device__ __forceinline__ void split8(float (&v)[8], u32x4 (&p)[3]) {
     for (int e = 0; e < 4; ++e) p[q][e] = cut_pair(v[2 * e], v[2 * e + 1]);
 #pragma unroll
   for (int e = 0; e < 4; ++e) p[2][e] = perm_b32(fbits(v[2 * e + 1]), fbits(v[2 * e]), 0x07060302u);
-}
-
-template <int J>
-__device__ __forceinline__ float row_lane(float v) {  // the value of lane 16 (l / 16) + J
-  return __uint_as_float(dpp_mov<0x150 + J>(fbits(v)));
-}
-template <int J>
-__device__ __forceinline__ void row_lanes(float v, float (&o)[16]) {
-  o[J] = row_lane<J>(v);
-  if constexpr (J + 1 < 16) row_lanes<J + 1>(v, o);
 }
 
 // One step's codes of a lane: the 8 bytes it stages or uses, their block

@@ -43,13 +43,6 @@ namespace {
 constexpr int kMN = 128, kMK = 64;
 constexpr int kMThreads = 256;
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef int v2i32 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) v2i32 lds_v2i32;
-typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-typedef __attribute__((address_space(3))) const f32x2 lds_f32x2_c;
-
 constexpr int kCopies = 8;               // of the level-pair table
 constexpr int kEntry = kCopies * 8;      // bytes from one byte value's pairs to the next
 constexpr int kEntryShift = 2;           // (byte << 8 | lane part) >> this: byte * kEntry + copy * 8
@@ -79,16 +72,6 @@ struct MidArgs {
   int k_splits, k_slab;  // slabs of K, and the K of one
   float* partials;       // [k_splits][M][N], or null
 };
-
-template <int J>
-__device__ __forceinline__ float row_lane(float v) {  // the value of lane 16 (l / 16) + J
-  return __uint_as_float(dpp_mov<0x150 + J>(__float_as_uint(v)));
-}
-template <int J>
-__device__ __forceinline__ void row_lanes(float v, float (&o)[16]) {
-  o[J] = row_lane<J>(v);
-  if constexpr (J + 1 < 16) row_lanes<J + 1>(v, o);
-}
 
 // NF4_LEVELS[c] for a per-lane c from immediates (no memory access)
 __device__ __forceinline__ float level_of(int c) {

@@ -642,23 +642,7 @@ hipError_t dispatch_w(const StripedArgs& a, int grid, int waves, bool xbf16, boo
 // before the MFMAs of the current one.  The waves' accumulators are added
 // through LDS in a fixed order.
 
-typedef int v2i32 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) v2i32 lds_v2i32;
-
-typedef __attribute__((address_space(3))) u32x2 lds_u32x2_w;
-
 constexpr int kSkStageOffset = kStripedSmem;  // after the level and DQ LUTs
-
-// the value of lane 16 (l / 16) + J, in every lane l
-template <int J>
-__device__ __forceinline__ float row_bcast(float v) {
-  return as_f(dpp_mov<0x150 + J>(as_u(v)));
-}
-template <int J>
-__device__ __forceinline__ void row_bcast_all(float v, float (&o)[16]) {
-  o[J] = row_bcast<J>(v);
-  if constexpr (J + 1 < 16) row_bcast_all<J + 1>(v, o);
-}
 
 template <int NT, int NW, int S, bool DQ, bool XF32>
 struct SkChunk {
@@ -711,7 +695,7 @@ __device__ __forceinline__ void sk_issue(SkChunk<NT, NW, S, DQ, XF32>& c, const 
 // 16 G + 2 m, 16 G + 2 m + 1 of this lane's column, m = 0..7).
 __device__ __forceinline__ void sk_lookup(f32x2 (&lv)[8], u32x2 code, uint32_t stage, uint32_t lane_off) {
   constexpr int kShift = kLutCopies == 32 ? 0 : (kLutCopies == 16 ? 1 : 2);
-  *reinterpret_cast<lds_u32x2_w*>((size_t)stage) = code;
+  *reinterpret_cast<lds_u32x2*>((size_t)stage) = code;
   const v2i32 nib = __builtin_amdgcn_ds_read_tr4_b64_v2i32(reinterpret_cast<lds_v2i32*>((size_t)stage));
 #pragma unroll
   for (int d = 0; d < 2; ++d)
@@ -830,7 +814,7 @@ __global__ __launch_bounds__(W * 64) void skinny_kernel(const void* x_arg, const
     for (int j = 0; j < D; ++j) {
       float sc[NW][16];
 #pragma unroll
-      for (int w = 0; w < NW; ++w) row_bcast_all<0>(sdec[j & 1][w], sc[w]);
+      for (int w = 0; w < NW; ++w) row_lanes<0>(sdec[j & 1][w], sc[w]);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int w = u / S, i = u % S;
