@@ -175,6 +175,7 @@ __global__ __launch_bounds__(kXaThreads) void lora_xa_kernel(const void* __restr
     }
   __syncthreads();
   static_assert(T * 64 <= kXaThreads, "one value a thread");
+  if (!SLABS && tid >= T * rank) return;
   const int t = tid / rank, c = tid % rank;
   const bool mine = t < T && m0 + t < M;
   const size_t at = (size_t)(m0 + t) * rank + c;
